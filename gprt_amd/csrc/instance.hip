@@ -867,7 +867,7 @@ GPRT_API void gprtSynthBounceRays(GPRTContext _ctx, GPRTAccel _a, GPRTBuffer _ra
   uint32_t *list = (uint32_t *)(b + al(scanBytes) + 2 * al((size_t)n * 4));
   const unsigned g = (n + 255) / 256;
   launch(ctx, s, "synth_hit_flags", k_hit_flags, dim3(g), dim3(256), 0, (const GPRTHit *)hits->d, n, flags);
-  scan_run(ctx, s, flags, offs, n, 0, false, state, nullptr);
+  scan_run(ctx, s, flags, offs, n, 0, false, state, nullptr, 0u);
   launch(ctx, s, "synth_hit_list", k_hit_list, dim3(g), dim3(256), 0, (const uint32_t *)flags,
          (const uint32_t *)offs, n, list);
   const bool inst = a->kind == AccelKind::Instances;

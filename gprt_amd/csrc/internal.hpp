@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <map>
@@ -70,6 +71,14 @@ struct SortConfig {
   int wavesPerCU = 0;    // LBVH sort passes: occupancy cap through LDS padding (0 = none)
 };
 
+// The scan family's look-back state of a context: tile statuses that count under one call's epoch
+// only, so nothing is cleared between calls.
+constexpr uint32_t kScanEpochs = (1u << 30) - 1u;
+struct ScanState {
+  uint64_t *words = nullptr;  // [0] total, [1] tile ticket, [2 + t] status of tile t
+  uint32_t tiles = 0, epoch = 0;
+};
+
 struct Context {
   SortConfig sortCfg;  // used by every sort and LBVH build issued on this context
   double syncTimeout = 6.0;  // seconds a host wait may take before it is reported (0: no limit)
@@ -86,8 +95,13 @@ struct Context {
   // Trace work counter (first 256 B) and per-lane stack spill area.
   void *traceScratch = nullptr;
   size_t traceBytes = 0;
-  // Small pinned host word for scan totals.
-  uint32_t *pinnedWord = nullptr;
+  // Pinned host word {sequence | total} that the scan kernels write, its device address, and the
+  // number of the call that wrote it last.
+  uint64_t *pinnedWord = nullptr, *pinnedWordDev = nullptr;
+  uint32_t scanSeq = 0;
+  ScanState scan;
+  // Event that host waits poll; a wait takes it for its duration.
+  std::atomic<hipEvent_t> waitEvent{nullptr};
   // Pool of triangle-accel descriptors (device, fixed capacity so addresses stay valid): the
   // address an instance record names (gprt::Instance::accelAddress) is a slot of this pool, which
   // lets the instance-accel build check every address on the device before reading through it.
@@ -266,8 +280,16 @@ size_t scan_scratch_bytes(size_t n);
 bool scan_noalloc_init(int device);
 void *scan_noalloc_state(int device);
 size_t scan_noalloc_max_items();
+// The total lands in the state's first word, and as {seq | total} in `hostWord` (device address of
+// host memory) when given. scan_run clears the state it is handed (scan_scratch_bytes); scan_run_kept
+// uses the context's own, which needs no clearing.
 void scan_run(Context *ctx, hipStream_t s, const uint32_t *in, uint32_t *out, size_t n, int mode, bool selectPositive,
-              void *scratch, uint32_t *totalDev);
+              void *state, uint64_t *hostWord, uint32_t seq);
+bool scan_run_kept(Context *ctx, hipStream_t s, const uint32_t *in, uint32_t *out, size_t n, int mode,
+                   bool selectPositive, uint64_t *hostWord, uint32_t seq);
+// The host word of a scan of n items is written behind the whole output (one tile), so that it is the
+// call's completion.
+bool scan_signals(size_t n, int mode);
 
 size_t sort_scratch_bytes(size_t n, int keyBits, int valBits, int loBit, int hiBit, const SortConfig &cfg);
 // Sorts n keys (keyBits 32|64) with optional payload (valBits 0|32|64) by key bits [loBit, hiBit).

@@ -374,7 +374,7 @@ float train_core(Context *ctx, Proposal *p, const void *rays, const void *hits, 
     hip_ok(hipMemcpyAsync(labels, userLabels, (size_t)count * 4, hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
   launch(ctx, s, "mlp_label_flags", k_label_flags, dim3(g), dim3(256), 0, (const int32_t *)labels, count,
          p->numClasses ? p->numClasses : (uint32_t)kMlpOut, flags);
-  scan_run(ctx, s, flags, offs, count, 0, false, scanState, nullptr);
+  scan_run(ctx, s, flags, offs, count, 0, false, scanState, nullptr, 0u);
   launch(ctx, s, "mlp_compact", k_compact, dim3(g), dim3(256), 0, (const GPRTRay *)rays, (const int32_t *)labels,
          (const uint32_t *)flags, (const uint32_t *)offs, count, cRays, cLabels);
   uint32_t labelled = 0;

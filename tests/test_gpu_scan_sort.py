@@ -100,6 +100,28 @@ def test_partition_select_random(ctx, orc, mode):
                                       ref[:total] if mode == "select" else ref)
 
 
+# Around the tiles (4,096, 16,384 and 45,056 items) and the sizes at which the tile changes, with no, all
+# and some items selected, the calls one after another on one context's state.
+@pytest.mark.parametrize("n", [1, 4095, 4096, 4097, 16383, 16384, 16385, 20481, (1 << 19) - 1, 1 << 19, (1 << 19) + 1,
+                               (6 << 20) - 3, 6 << 20, (6 << 20) + 5])
+def test_scan_family_tiles(ctx, n):
+    rng = np.random.default_rng(n)
+    some = rng.integers(-2**31, 2**31, n, dtype=np.int64).astype(np.int32)
+    for x in (some, np.abs(some) % 1000, -1 - np.abs(some) % 1000):
+        sel, rest = x[x >= 0], x[x < 0]
+        out, total = _scan(ctx, x, "partition")
+        assert total == len(sel)
+        np.testing.assert_array_equal(out, np.concatenate([sel, rest[::-1]]))
+        out, total = _scan(ctx, x, "select", sel_pos=False, scratch=None)
+        assert total == len(rest)
+        np.testing.assert_array_equal(out[:total], rest)
+    c = np.cumsum(some.view(np.uint32), dtype=np.uint64)
+    out, total = _scan(ctx, some.view(np.uint32), "sum", scratch=None)
+    assert total == int(c[-1]) & 0xFFFFFFFF
+    assert out[0] == 0
+    np.testing.assert_array_equal(out[1:], (c[:-1] & np.uint64(0xFFFFFFFF)).astype(np.uint32))
+
+
 def test_exclusive_sum_full_size(ctx):
     # 2^28 u32 uniform in [0, 255]: the exclusive-scan microbenchmark size; the sum wraps.
     n = 1 << 28
