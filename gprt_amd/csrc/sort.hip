@@ -14,6 +14,8 @@
 //  * ping-pong buffers are picked on the device from the active-pass mask, and k_final_copy
 //    moves the result back when an odd number of passes ran — no host round trip, so the whole
 //    sort can be captured in a hipGraph.
+// Up to 16,384 keys, where those launches would be all the time there is, k_rank places every key by
+// comparing it with all others and k_copy_pairs puts the result back: two launches.
 #include "device_common.hpp"
 #include "internal.hpp"
 
@@ -372,8 +374,90 @@ __global__ void __launch_bounds__(256) k_final_copy(KT *__restrict__ keys0, cons
 }
 
 // ------------------------------------------------------------------------------------------------
+// Small sorts: every key's rank by comparing it with every key.
+// ------------------------------------------------------------------------------------------------
+// One workgroup per 64 keys (lane = key); its 16 waves share the comparisons with all keys, 16 keys
+// at a time. Those are uniform over the wave and come through scalar loads, so a pair costs one compare
+// and one add with carry. The rank (ties by index: stable) is the key's place in `outKeys`. The
+// workgroup's own keys and the last n % 16 are compared from registers.
+template <typename KT>
+__device__ __forceinline__ KT read_lane(KT k, uint32_t lane) {
+  if constexpr (sizeof(KT) == 8)
+    return (KT)wave_read((uint32_t)(k >> 32), (int)lane) << 32 | wave_read((uint32_t)k, (int)lane);
+  else
+    return wave_read(k, (int)lane);
+}
+
+template <typename KT, int VB>
+__global__ void __launch_bounds__(1024)
+    k_rank(const KT *__restrict__ keys, const void *__restrict__ vals, KT *__restrict__ outKeys,
+           void *__restrict__ outVals, uint32_t n) {
+  using VT = typename ValType<VB>::T;
+  constexpr uint32_t W = 16, C = 128 / sizeof(KT);
+  __shared__ uint32_t s_count[W][64];
+  const uint32_t l = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t i0 = blockIdx.x * 64u, i = min(i0 + l, n - 1);
+  const KT k = keys[i];
+  VT v = 0;
+  if (VB && w == 0) v = ((const VT *)vals)[i];
+  const uint32_t chunks = n / C, own = i0 / C;
+  const KT tail = keys[min(chunks * C + l, n - 1)];
+  uint32_t count = 0;
+  for (uint32_t c = w; c < min(own, chunks); c += W) {
+#pragma unroll
+    for (uint32_t x = 0; x < C; ++x) count += keys[c * C + x] <= k ? 1u : 0u;
+  }
+  for (uint32_t c = own + 64u / C + w; c < chunks; c += W) {
+#pragma unroll
+    for (uint32_t x = 0; x < C; ++x) count += keys[c * C + x] < k ? 1u : 0u;
+  }
+  if (w == W - 1 && chunks * C >= i0 + 64u) {
+    for (uint32_t x = 0; x < n - chunks * C; ++x) count += read_lane(tail, x) < k ? 1u : 0u;
+  }
+#pragma unroll
+  for (uint32_t y = 0; y < 64u / W; ++y) {
+    const uint32_t x = w * (64u / W) + y;
+    const KT o = read_lane(k, x);
+    if (i0 + x < n) count += (o < k || (o == k && x < l)) ? 1u : 0u;
+  }
+  s_count[w][l] = count;
+  __syncthreads();
+  if (w == 0 && i0 + l < n) {
+    uint32_t rank = 0;
+#pragma unroll
+    for (uint32_t x = 0; x < W; ++x) rank += s_count[x][l];
+    outKeys[rank] = k;
+    if (VB) ((VT *)outVals)[rank] = v;
+  }
+}
+
+template <typename KT, int VB>
+__global__ void __launch_bounds__(256) k_copy_pairs(const KT *__restrict__ keys, const void *__restrict__ vals,
+                                                    KT *__restrict__ outKeys, void *__restrict__ outVals, uint32_t n) {
+  using VT = typename ValType<VB>::T;
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  outKeys[i] = keys[i];
+  if (VB) ((VT *)outVals)[i] = ((const VT *)vals)[i];
+}
+
+// ------------------------------------------------------------------------------------------------
 // Host dispatch
 // ------------------------------------------------------------------------------------------------
+// Up to here ranks beat the radix passes, whose 8 to 12 dependent launches take 6 to 10 us each however
+// few keys there are (a copy of the keys and the sort, us, 64-bit pairs / 32-bit keys, ranks against
+// passes): 3,000 keys 13 against 89 / 13 against 41, 16,000 keys 40 against 124 / 38 against 49; 24,000
+// keys 95 against 129 / 93 against 49, as the compares grow with the square.
+constexpr size_t kRankSortMax = 16384;
+
+template <typename KT, int VB>
+void run_rank(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAlt, void *valsAlt, size_t n) {
+  launch(ctx, s, "sort_rank", k_rank<KT, VB>, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, (const KT *)keys,
+         (const void *)vals, (KT *)keysAlt, valsAlt, (uint32_t)n);
+  launch(ctx, s, "sort_rank_copy", k_copy_pairs<KT, VB>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+         (const KT *)keysAlt, (const void *)valsAlt, (KT *)keys, vals, (uint32_t)n);
+}
+
 inline int passes_for(int loBit, int hiBit, int bits) { return (hiBit - loBit + bits - 1) / bits; }
 
 // Keys per tile of one sort: 2,048 when asked for; 4,096 for 64-bit keys or payloads (their
@@ -446,6 +530,10 @@ bool run_bits(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAlt
 template <typename KT, int VB>
 bool run_kv(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAlt, void *valsAlt, size_t n, int loBit,
             int hiBit, void *scratch, const SortConfig &cfg) {
+  if (n <= kRankSortMax && loBit == 0 && hiBit == (int)sizeof(KT) * 8) {
+    run_rank<KT, VB>(ctx, s, keys, vals, keysAlt, valsAlt, n);
+    return true;
+  }
   switch (cfg.digitBits) {
     case 4: return run_bits<KT, VB, 4>(ctx, s, keys, vals, keysAlt, valsAlt, n, loBit, hiBit, scratch, cfg);
     case 6: return run_bits<KT, VB, 6>(ctx, s, keys, vals, keysAlt, valsAlt, n, loBit, hiBit, scratch, cfg);

@@ -223,6 +223,24 @@ def test_sort_edge_sizes(ctx, orc, n):
     np.testing.assert_array_equal(v, rv)
 
 
+# Around the 16-key chunks, the 64 keys of a workgroup and the largest size of the sort by ranks, with
+# duplicates that the payload's order tells apart and keys that equal the largest value.
+@pytest.mark.parametrize("kdt,vdt", [(np.uint32, np.uint32), (np.uint64, np.uint64), (np.uint64, np.uint32),
+                                     (np.uint32, None), (np.uint64, None)])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 33, 63, 64, 65, 127, 128, 129, 1000, 5003, 16383, 16384, 16385])
+def test_sort_by_ranks(ctx, n, kdt, vdt):
+    rng = np.random.default_rng(n)
+    top = np.iinfo(kdt).max
+    keys = rng.integers(0, max(2, n // 3), n).astype(kdt) * kdt(top // max(2, n // 3))
+    keys[::5] = top
+    vals = None if vdt is None else np.arange(n, dtype=vdt)
+    k, v = _sort_kv(ctx, keys, vals)
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(k, keys[order])
+    if vals is not None:
+        np.testing.assert_array_equal(v, vals[order])
+
+
 def test_sort_constant_and_single_digit_keys(ctx, orc):
     n = 50_000
     # every digit constant: all passes skipped, data untouched
