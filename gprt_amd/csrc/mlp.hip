@@ -27,44 +27,16 @@
 #include "bvh.hpp"
 #include "device_common.hpp"
 #include "internal.hpp"
-#include "mlp.hpp"
+#include "mlp_device.hpp"
 
 namespace gprt {
 
 namespace {
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
-
-union Frag {
-  bf16x8_t v;
-  uint4 u;
-  uint16_t h[8];
-};
-
-__device__ __forceinline__ f32x4_t mfma16(const Frag &a, const Frag &b, f32x4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, c, 0, 0, 0);
-}
-
-// FP32 -> bf16 with round-to-nearest-even (NaN stays NaN).
-__host__ __device__ __forceinline__ uint16_t f2bf(float f) {
-  union {
-    float f;
-    uint32_t u;
-  } x;
-  x.f = f;
-  if ((x.u & 0x7FFFFFFFu) > 0x7F800000u) return (uint16_t)((x.u >> 16) | 0x40u);
-  const uint32_t r = 0x7FFFu + ((x.u >> 16) & 1u);
-  return (uint16_t)((x.u + r) >> 16);
-}
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-
 // ------------------------------------------------------------------------------------------------
 // Input encoding, produced directly as 64 packed words (two bf16 per word, low half first):
 // words 0..2 = (o.x,o.y) (o.z,d.x) (d.y,d.z); word 3 + 8c + k = (sin, cos)(2^k pi v_c); rest 0.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) { return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16); }
-
 __device__ __forceinline__ void encode_ray(const GPRTRay &r, uint32_t (&wds)[kMlpInPad / 2]) {
   const float v[6] = {r.ox, r.oy, r.oz, r.dx, r.dy, r.dz};
   wds[0] = pack2(v[0], v[1]);
@@ -101,105 +73,32 @@ __global__ void __launch_bounds__(256) k_encode(const GPRTRay *__restrict__ rays
 }
 
 // ------------------------------------------------------------------------------------------------
-// Generic bf16 GEMM on MFMA 16x16x32 with FP32 accumulation:
-//   C[m][n] = alpha * sum_k A(m,k) B(k,n) (+ bias[n]) (* (mask(m,n) > 0)) (relu) (+= C)
-// A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn]: any transposition through strides.
-// Workgroup tile 64x64 (4 waves of 32x32 = 2x2 MFMA tiles), K step 64 staged in LDS. Each operand
-// is read 16 bytes at a time along whichever of its strides is 1 (K-contiguous rows are copied,
-// M/N-contiguous columns are transposed into LDS); other layouts, unaligned operands and tile
-// edges use element loads. Split K (split > 1): workgroup z covers the K range
-// [z*kPer, (z+1)*kPer) and writes its partial sums to ws[z][M][N]; k_gemm_reduce adds the splits
-// in order and applies the epilogue, so the result does not depend on scheduling.
+// A layer of a batch (gprtProposalLogits): C = A B^T + bias, bf16 operands with contiguous K = 128, FP32
+// accumulation, on MFMA 16x16x32. Workgroup tile 64x64 (4 waves of 32x32 = 2x2 MFMA tiles), K steps of
+// 64 staged in LDS.
 // ------------------------------------------------------------------------------------------------
 struct GemmArgs {
-  const uint16_t *A;
-  long long sam, sak;
-  const uint16_t *B;
-  long long sbk, sbn;
-  float *Cf;
-  uint16_t *Cb;
-  long long scm, scn;
-  int M, N, K;
+  const uint16_t *A, *B;  // [M][128], [N][128]
+  float *Cf;              // C in fp32, or
+  uint16_t *Cb;           // relu(C) in bf16
+  int M, N;
   const float *bias;
-  const uint16_t *mask;
-  long long smm, smn;
-  int relu;
-  int accumulate;
-  float alpha;
-  int aMode, bMode;  // 0: element loads; 1: K-contiguous 16-byte loads; 2: M/N-contiguous 16-byte loads
-  int split, kPer;
-  float *ws;
 };
 
 constexpr int kGK = 64;    // K step
 constexpr int kGPad = 72;  // LDS row length in elements (16-byte aligned rows)
+static_assert(kMlpInPad == kMlpHid && kMlpHid % kGK == 0, "every layer's K is 128");
 
-// S[row][k] = P(r0 + row, k0 + k) for a 64 x 64 block, where P(r, k) = P[r*srow + k*sk], zero
-// outside [0, rows) x [k0, kEnd).
-__device__ __forceinline__ void gemm_stage(const uint16_t *__restrict__ P, long long srow, long long sk, int mode,
-                                           int rows, int r0, int k0, int kEnd, uint16_t (*S)[kGPad], int tid) {
-  if (mode == 1) {
+// S[row][k] = P[r0 + row][k0 + k] for a 64 x 64 block, zero past `rows`.
+__device__ __forceinline__ void gemm_stage(const uint16_t *__restrict__ P, int rows, int r0, int k0,
+                                           uint16_t (*S)[kGPad], int tid) {
 #pragma unroll
-    for (int c = tid; c < 512; c += 256) {
-      const int row = c >> 3, kc = (c & 7) * 8;
-      const int r = r0 + row, k = k0 + kc;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (r < rows && k + 8 <= kEnd) {
-        v = *(const uint4 *)(P + (long long)r * srow + k);
-      } else if (r < rows) {
-        uint16_t e[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) e[j] = k + j < kEnd ? P[(long long)r * srow + k + j] : (uint16_t)0;
-        v = make_uint4(e[0] | (uint32_t)e[1] << 16, e[2] | (uint32_t)e[3] << 16, e[4] | (uint32_t)e[5] << 16,
-                       e[6] | (uint32_t)e[7] << 16);
-      }
-      *(uint4 *)&S[row][kc] = v;
-    }
-  } else if (mode == 2) {
-#pragma unroll
-    for (int c = tid; c < 512; c += 256) {
-      const int kk = c >> 3, rc = (c & 7) * 8;
-      const int r = r0 + rc, k = k0 + kk;
-      uint16_t e[8];
-      if (k < kEnd && r + 8 <= rows) {
-        const uint4 v = *(const uint4 *)(P + r + (long long)k * sk);
-        const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          e[2 * j] = (uint16_t)(w4[j] & 0xFFFFu);
-          e[2 * j + 1] = (uint16_t)(w4[j] >> 16);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) e[j] = (k < kEnd && r + j < rows) ? P[r + j + (long long)k * sk] : (uint16_t)0;
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) S[rc + j][kk] = e[j];
-    }
-  } else {
-    const int row = tid >> 2, kq = (tid & 3) * 16;
-    const int r = r0 + row;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int k = k0 + kq + j;
-      S[row][kq + j] = (r < rows && k < kEnd) ? P[(long long)r * srow + (long long)k * sk] : (uint16_t)0;
-    }
+  for (int c = tid; c < 512; c += 256) {
+    const int row = c >> 3, kc = (c & 7) * 8;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (r0 + row < rows) v = *(const uint4 *)(P + (size_t)(r0 + row) * kMlpHid + k0 + kc);
+    *(uint4 *)&S[row][kc] = v;
   }
-}
-
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs &g, int m, int n, float sum) {
-  float v = g.alpha * sum;
-  if (g.bias) v += g.bias[n];
-  if (g.mask && !(bf2f(g.mask[(long long)m * g.smm + (long long)n * g.smn]) > 0.f)) v = 0.f;
-  if (g.relu) v = fmaxf(v, 0.f);
-  const long long o = (long long)m * g.scm + (long long)n * g.scn;
-  if (g.Cf) {
-    if (g.accumulate)
-      g.Cf[o] += v;
-    else
-      g.Cf[o] = v;
-  }
-  if (g.Cb) g.Cb[o] = f2bf(v);
 }
 
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
@@ -208,15 +107,14 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-  const int kBeg = blockIdx.z * g.kPer, kEnd = min(g.K, kBeg + g.kPer);
   f32x4_t acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = kBeg; k0 < kEnd; k0 += kGK) {
-    gemm_stage(g.A, g.sam, g.sak, g.aMode, g.M, m0, k0, kEnd, As, tid);
-    gemm_stage(g.B, g.sbn, g.sbk, g.bMode, g.N, n0, k0, kEnd, Bs, tid);
+  for (int k0 = 0; k0 < kMlpHid; k0 += kGK) {
+    gemm_stage(g.A, g.M, m0, k0, As, tid);
+    gemm_stage(g.B, g.N, n0, k0, Bs, tid);
     __syncthreads();
 #pragma unroll
     for (int ks = 0; ks < kGK; ks += 32) {
@@ -242,179 +140,11 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
         const int m = m0 + wm + i * 16 + 4 * (l >> 4) + q;
         const int n = n0 + wn + j * 16 + (l & 15);
         if (m >= g.M || n >= g.N) continue;
-        if (g.split > 1)
-          g.ws[((long long)blockIdx.z * g.M + m) * g.N + n] = acc[i][j][q];
-        else
-          gemm_epilogue(g, m, n, acc[i][j][q]);
+        const float v = acc[i][j][q] + g.bias[n];
+        const size_t o = (size_t)m * g.N + n;
+        if (g.Cf) g.Cf[o] = v;
+        if (g.Cb) g.Cb[o] = f2bf(fmaxf(v, 0.f));
       }
-}
-
-// Sums the split-K partials in split order, then applies the epilogue.
-__global__ void __launch_bounds__(256) k_gemm_reduce(GemmArgs g) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long mn = (long long)g.M * g.N;
-  if (i >= mn) return;
-  float sum = 0.f;
-  for (int z = 0; z < g.split; ++z) sum += g.ws[z * mn + i];
-  gemm_epilogue(g, (int)(i / g.N), (int)(i % g.N), sum);
-}
-
-// ------------------------------------------------------------------------------------------------
-// Softmax cross-entropy gradient: dZ = (softmax(z) - onehot(y)) * scale; rows with y < 0 give 0.
-// One workgroup per row. loss += -log softmax(z)[y] * scale.
-// ------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_softmax_ce(const float *__restrict__ Z, const int32_t *__restrict__ labels,
-                                                    uint16_t *__restrict__ dZ, float scale, float *__restrict__ loss,
-                                                    uint32_t *__restrict__ correct) {
-  static_assert(kMlpOut == 4096, "one row is 16 logits per thread");
-  const uint32_t row = blockIdx.x;
-  const int tid = threadIdx.x;
-  const float *z = Z + (size_t)row * kMlpOut;
-  uint16_t *dz = dZ + (size_t)row * kMlpOut;
-  const int y = labels[row];
-  __shared__ float s_red[4];
-  __shared__ int s_idx[4];
-  // The row is read once: thread tid holds logits j*1024 + 4*tid + q (increasing with j, q).
-  float v[16];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float4 f = *(const float4 *)(z + j * 1024 + 4 * tid);
-    v[4 * j] = f.x;
-    v[4 * j + 1] = f.y;
-    v[4 * j + 2] = f.z;
-    v[4 * j + 3] = f.w;
-  }
-  float mx = -INFINITY;
-  int amx = 0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (v[i] > mx) {
-      mx = v[i];
-      amx = (i >> 2) * 1024 + 4 * tid + (i & 3);
-    }
-  }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    const float om = __shfl_xor(mx, o, 64);
-    const int oi = __shfl_xor(amx, o, 64);
-    if (om > mx || (om == mx && oi < amx)) {
-      mx = om;
-      amx = oi;
-    }
-  }
-  if ((tid & 63) == 0) {
-    s_red[tid >> 6] = mx;
-    s_idx[tid >> 6] = amx;
-  }
-  __syncthreads();
-  mx = s_red[0];
-  amx = s_idx[0];
-  for (int w = 1; w < 4; ++w)
-    if (s_red[w] > mx || (s_red[w] == mx && s_idx[w] < amx)) {
-      mx = s_red[w];
-      amx = s_idx[w];
-    }
-  __syncthreads();
-  float e[16], sum = 0.f;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    e[i] = expf(v[i] - mx);
-    sum += e[i];
-  }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-  if ((tid & 63) == 0) s_red[tid >> 6] = sum;
-  __syncthreads();
-  sum = s_red[0] + s_red[1] + s_red[2] + s_red[3];
-  const float inv = 1.0f / sum;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    uint16_t o[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int c = j * 1024 + 4 * tid + q;
-      const float g = y >= 0 ? (e[4 * j + q] * inv - (c == y ? 1.f : 0.f)) * scale : 0.f;
-      o[q] = f2bf(g);
-    }
-    *(uint2 *)(dz + j * 1024 + 4 * tid) = make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
-  }
-  if (tid == 0 && y >= 0) {
-    atomicAdd(loss, (logf(sum) + mx - z[y]) * scale);
-    if (amx == y) atomicAdd(correct, 1u);
-  }
-}
-
-// Column sums (bias gradients), deterministic in two passes: k_colsum_part sums a chunk of rows
-// for 64 columns per workgroup (8 columns per thread with 16-byte loads when `vec`; 32 row lanes
-// reduced in LDS in a fixed order) into part[chunk][n]; k_colsum_fin adds the chunks in order.
-__global__ void __launch_bounds__(256) k_colsum_part(const uint16_t *__restrict__ A, int M, int N, int lda,
-                                                     int rowsPerChunk, int vec, float *__restrict__ part) {
-  __shared__ float s[32][65];
-  const int cg = threadIdx.x & 7, rl = threadIdx.x >> 3;
-  const int n0 = blockIdx.x * 64 + cg * 8;
-  const int mBeg = blockIdx.y * rowsPerChunk, mEnd = min(M, mBeg + rowsPerChunk);
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int m = mBeg + rl; m < mEnd; m += 32) {
-    const uint16_t *row = A + (size_t)m * lda;
-    if (vec && n0 + 8 <= N) {
-      const uint4 u = *(const uint4 *)(row + n0);
-      const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        acc[2 * j] += bf2f((uint16_t)(w4[j] & 0xFFFFu));
-        acc[2 * j + 1] += bf2f((uint16_t)(w4[j] >> 16));
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (n0 + j < N) acc[j] += bf2f(row[n0 + j]);
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) s[rl][cg * 8 + j] = acc[j];
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    float t = 0.f;
-    for (int r = 0; r < 32; ++r) t += s[r][threadIdx.x];
-    const int n = blockIdx.x * 64 + threadIdx.x;
-    if (n < N) part[(size_t)blockIdx.y * N + n] = t;
-  }
-}
-
-__global__ void __launch_bounds__(256) k_colsum_fin(const float *__restrict__ part, int chunks, int N,
-                                                    float *__restrict__ out) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float t = 0.f;
-  for (int c = 0; c < chunks; ++c) t += part[(size_t)c * N + n];
-  out[n] = t;
-}
-
-// Adam (bias-corrected) on the fp32 parameters; refreshes the bf16 weight copies.
-__global__ void __launch_bounds__(256) k_adam(float *__restrict__ w, const float *__restrict__ g,
-                                              float *__restrict__ m, float *__restrict__ v, uint32_t n, float lr,
-                                              float b1, float b2, float eps, float c1, float c2,
-                                              const uint32_t *__restrict__ bfMap, uint16_t *__restrict__ wbf) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float mh = mi / c1, vh = vi / c2;
-  const float wi = w[i] - lr * mh / (sqrtf(vh) + eps);
-  w[i] = wi;
-  const uint32_t b = bfMap[i];
-  if (b != 0xFFFFFFFFu) wbf[b] = f2bf(wi);
-}
-
-__global__ void __launch_bounds__(256) k_to_bf16(const float *__restrict__ w, const uint32_t *__restrict__ bfMap,
-                                                 uint16_t *__restrict__ wbf, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t b = bfMap[i];
-  if (b != 0xFFFFFFFFu) wbf[b] = f2bf(w[i]);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -735,61 +465,6 @@ __global__ void __launch_bounds__(256) k_labels_of_leaves(const int32_t *__restr
 
 unsigned blocks_for(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 
-// out[n] = sum over the M rows of A (bf16, row stride lda), through the GEMM workspace.
-void colsum(Context *ctx, hipStream_t s, const uint16_t *A, int M, int N, int lda, float *out, const Proposal *p) {
-  int rows = 256;
-  while ((size_t)((M + rows - 1) / rows) * N * 4 > p->gemmWsBytes) rows *= 2;
-  const int chunks = std::max(1, (M + rows - 1) / rows);
-  const int vec = ((uintptr_t)A & 15u) == 0 && lda % 8 == 0;
-  launch(ctx, s, "mlp_colsum", k_colsum_part, dim3((N + 63) / 64, chunks), dim3(256), 0, A, M, N, lda, rows, vec,
-         p->gemmWs);
-  launch(ctx, s, "mlp_colsum", k_colsum_fin, dim3(blocks_for(N, 256)), dim3(256), 0, (const float *)p->gemmWs, chunks,
-         N, out);
-}
-
-// Picks each operand's load mode and the K split, then launches (and reduces the splits).
-void gemm(Context *ctx, hipStream_t s, GemmArgs g, const char *name, const Proposal *p) {
-  auto vec_ok = [](const void *ptr, long long otherStride) {
-    return ((uintptr_t)ptr & 15u) == 0 && otherStride % 8 == 0;
-  };
-  g.aMode = (g.sak == 1 && vec_ok(g.A, g.sam)) ? 1 : (g.sam == 1 && vec_ok(g.A, g.sak)) ? 2 : 0;
-  g.bMode = (g.sbk == 1 && vec_ok(g.B, g.sbn)) ? 1 : (g.sbn == 1 && vec_ok(g.B, g.sbk)) ? 2 : 0;
-  const long long tiles = (long long)((g.N + 63) / 64) * ((g.M + 63) / 64);
-  // Few output tiles over a long K (weight gradients): split K so ~512 workgroups run, each over
-  // at least 256 of K, as far as the workspace holds the partials.
-  int split = 1;
-  if (tiles < 256 && g.K >= 512 && p->gemmWs) {
-    split = (int)std::min<long long>(std::max<long long>(512 / tiles, 1), g.K / 256);
-    while (split > 1 && (size_t)split * g.M * g.N * 4 > p->gemmWsBytes) --split;
-  }
-  g.kPer = ((g.K + split - 1) / split + kGK - 1) / kGK * kGK;
-  g.split = (g.K + g.kPer - 1) / g.kPer;
-  if (g.split < 1) g.split = 1;
-  g.ws = p->gemmWs;
-  dim3 grid((g.N + 63) / 64, (g.M + 63) / 64, g.split);
-  launch(ctx, s, name, k_gemm, grid, dim3(256), 0, g);
-  if (g.split > 1)
-    launch(ctx, s, "mlp_gemm_reduce", k_gemm_reduce, dim3((unsigned)(((long long)g.M * g.N + 255) / 256)), dim3(256),
-           0, g);
-}
-
-GemmArgs gemm_args(const uint16_t *A, long long sam, long long sak, const uint16_t *B, long long sbk, long long sbn,
-                   int M, int N, int K) {
-  GemmArgs g;
-  std::memset(&g, 0, sizeof(g));
-  g.A = A;
-  g.sam = sam;
-  g.sak = sak;
-  g.B = B;
-  g.sbk = sbk;
-  g.sbn = sbn;
-  g.M = M;
-  g.N = N;
-  g.K = K;
-  g.alpha = 1.f;
-  return g;
-}
-
 }  // namespace
 
 // ------------------------------------------------------------------------------------------------
@@ -799,41 +474,19 @@ size_t mlp_param_count() { return kMlpParams; }
 
 bool mlp_alloc(Context *ctx, Proposal *p, uint32_t maxBatch) {
   (void)ctx;
-  auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-  const size_t P = kMlpParams;
+  const size_t P = kMlpParams, B = maxBatch;
+  const TrainBytes train = mlp_train_bytes(maxBatch);
   size_t off = 0;
-  const size_t oW = off;
-  off += al(P * 4);
-  const size_t oG = off;
-  off += al(P * 4);
-  const size_t oM = off;
-  off += al(P * 4);
-  const size_t oV = off;
-  off += al(P * 4);
-  const size_t oMap = off;
-  off += al(P * 4);
-  const size_t oBf = off;
-  off += al(kMlpWeights * 2);
-  const size_t oBias = off;
-  off += al(kMlpBiases * 4);
-  const size_t oStat = off;
-  off += al(64);
-  const size_t B = maxBatch;
-  const size_t oX = off;
-  off += al(B * kMlpInPad * 2);
-  const size_t oH = off;
-  off += al(3 * B * kMlpHid * 2);
-  const size_t oD = off;
-  off += al(3 * B * kMlpHid * 2);
-  const size_t oZ = off;
-  off += al(B * kMlpOut * 4);
-  const size_t oDZ = off;
-  off += al(B * kMlpOut * 2);
-  const size_t oL = off;
-  off += al(B * 4);
-  const size_t oWs = off;  // split-K partial sums of the training GEMMs
-  const size_t wsBytes = (size_t)16 << 20;
-  off += al(wsBytes);
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t oW = take(P * 4), oG = take(P * 4), oM = take(P * 4), oV = take(P * 4);
+  const size_t oRows = take(kMlpWeights * 2), oFwd = take(kMlpWeights * 2), oBwd = take(kMlpWeights * 2);
+  const size_t oBias = take(kMlpBiases * 4), oStat = take(64);
+  const size_t oX = take(B * kMlpInPad * 2), oH = take(3 * B * kMlpHid * 2), oZ = take(B * kMlpOut * 4);
+  const size_t oAct = take(train.act), oDZ = take(train.dz), oLoss = take(train.loss), oWs = take(train.ws);
   if (!hip_ok(hipMalloc(&p->block, off), "hipMalloc(proposal)")) return false;
   p->blockBytes = off;
   char *b = (char *)p->block;
@@ -841,26 +494,16 @@ bool mlp_alloc(Context *ctx, Proposal *p, uint32_t maxBatch) {
   p->g = (float *)(b + oG);
   p->m = (float *)(b + oM);
   p->v = (float *)(b + oV);
-  p->bfMap = (uint32_t *)(b + oMap);
-  p->wbf = (uint16_t *)(b + oBf);
-  p->bias = (float *)(b + oBias);
+  p->weights = MlpWeights{(uint16_t *)(b + oRows), (uint16_t *)(b + oFwd), (uint16_t *)(b + oBwd), (float *)(b + oBias)};
   p->stats = (float *)(b + oStat);
   p->X = (uint16_t *)(b + oX);
   p->H = (uint16_t *)(b + oH);
-  p->dA = (uint16_t *)(b + oD);
   p->Z = (float *)(b + oZ);
+  p->act = (uint16_t *)(b + oAct);
   p->dZ = (uint16_t *)(b + oDZ);
-  p->labels = (int32_t *)(b + oL);
-  p->gemmWs = (float *)(b + oWs);
-  p->gemmWsBytes = wsBytes;
+  p->rowLoss = (float *)(b + oLoss);
+  p->trainWs = (float *)(b + oWs);
   p->maxBatch = maxBatch;
-  // Map from flat fp32 parameter index to its bf16 copy (weights only).
-  std::vector<uint32_t> map(P, 0xFFFFFFFFu);
-  for (int layer = 0; layer < 4; ++layer) {
-    const size_t wOff = mlp_weight_offset(layer), n = mlp_weight_size(layer), bfOff = mlp_bf16_offset(layer);
-    for (size_t i = 0; i < n; ++i) map[wOff + i] = (uint32_t)(bfOff + i);
-  }
-  if (!hip_ok(hipMemcpy(p->bfMap, map.data(), P * 4, hipMemcpyHostToDevice), "hipMemcpy(bfMap)")) return false;
   return true;
 }
 
@@ -870,112 +513,31 @@ void mlp_release(Proposal *p) {
   p->block = p->treeBlock = nullptr;
 }
 
-// Copies fp32 parameters to the device and refreshes the bf16 weights and the bias vector.
+// Copies fp32 parameters to the device, refreshes the bf16 weights and the bias vector and resets Adam.
 bool mlp_set_params(Context *ctx, hipStream_t s, Proposal *p, const float *host) {
   if (!hip_ok(hipMemcpyAsync(p->w, host, kMlpParams * 4, hipMemcpyHostToDevice, s), "hipMemcpyAsync(params)"))
     return false;
-  launch(ctx, s, "mlp_to_bf16", k_to_bf16, dim3(blocks_for(kMlpParams, 256)), dim3(256), 0, (const float *)p->w,
-         (const uint32_t *)p->bfMap, p->wbf, (uint32_t)kMlpParams);
+  mlp_store_params(ctx, s, p);
   fill_u32(ctx, s, p->m, 0u, kMlpParams);
   fill_u32(ctx, s, p->v, 0u, kMlpParams);
   p->step = 0;
-  return mlp_refresh_bias(ctx, s, p);
-}
-
-bool mlp_refresh_bias(Context *ctx, hipStream_t s, Proposal *p) {
-  (void)ctx;
-  for (int layer = 0; layer < 4; ++layer) {
-    const size_t n = layer < 3 ? kMlpHid : kMlpOut;
-    if (!hip_ok(hipMemcpyAsync(p->bias + layer * kMlpHid, p->w + mlp_bias_offset(layer), n * 4,
-                               hipMemcpyDeviceToDevice, s),
-                "hipMemcpyAsync(bias)"))
-      return false;
-  }
   return true;
 }
 
-const uint16_t *mlp_wbf(const Proposal *p, int layer) { return p->wbf + mlp_bf16_offset(layer); }
+const uint16_t *mlp_wbf(const Proposal *p, int layer) { return p->weights.rows + mlp_bf16_offset(layer); }
 
-// Forward of a batch with stored activations (training / logits). Z gets the fp32 logits.
+// Forward of a batch with stored activations. Z gets the fp32 logits.
 void mlp_forward_batch(Context *ctx, hipStream_t s, Proposal *p, const void *rays, uint32_t n) {
   launch(ctx, s, "mlp_encode", k_encode, dim3(blocks_for(n, 256)), dim3(256), 0, (const GPRTRay *)rays, n, p->X);
   const uint16_t *in = p->X;
-  int inStride = kMlpInPad;
-  for (int layer = 0; layer < 3; ++layer) {
-    uint16_t *out = p->H + (size_t)layer * p->maxBatch * kMlpHid;
-    GemmArgs g = gemm_args(in, inStride, 1, mlp_wbf(p, layer), 1, kMlpInPad, (int)n, kMlpHid, kMlpInPad);
-    g.Cb = out;
-    g.scm = kMlpHid;
-    g.scn = 1;
-    g.bias = p->w + mlp_bias_offset(layer);
-    g.relu = 1;
-    gemm(ctx, s, g, "mlp_gemm_fwd", p);
+  for (int layer = 0; layer < 4; ++layer) {
+    uint16_t *out = layer < 3 ? p->H + (size_t)layer * p->maxBatch * kMlpHid : nullptr;
+    const int N = layer < 3 ? kMlpHid : kMlpOut;
+    const GemmArgs g{in, mlp_wbf(p, layer), layer < 3 ? nullptr : p->Z, out, (int)n, N,
+                     p->weights.bias + layer * kMlpHid};
+    launch(ctx, s, "mlp_gemm_fwd", k_gemm, dim3((unsigned)(N / 64), (n + 63) / 64), dim3(256), 0, g);
     in = out;
-    inStride = kMlpHid;
   }
-  GemmArgs g = gemm_args(in, kMlpHid, 1, mlp_wbf(p, 3), 1, kMlpHid, (int)n, kMlpOut, kMlpHid);
-  g.Cf = p->Z;
-  g.scm = kMlpOut;
-  g.scn = 1;
-  g.bias = p->w + mlp_bias_offset(3);
-  gemm(ctx, s, g, "mlp_gemm_fwd", p);
-}
-
-// Gradients of the mean cross-entropy over the labelled rays of one batch (into p->g).
-void mlp_backward_batch(Context *ctx, hipStream_t s, Proposal *p, uint32_t n, uint32_t labelled) {
-  const float scale = labelled ? 1.0f / (float)labelled : 0.f;
-  fill_u32(ctx, s, p->g, 0u, kMlpParams);  // each gradient entry is then written exactly once
-  launch(ctx, s, "mlp_softmax_ce", k_softmax_ce, dim3(n), dim3(256), 0, (const float *)p->Z,
-         (const int32_t *)p->labels, p->dZ, scale, p->stats, (uint32_t *)(p->stats + 1));
-  const size_t B = p->maxBatch;
-  const uint16_t *H[3] = {p->H, p->H + B * kMlpHid, p->H + 2 * B * kMlpHid};
-  // Output layer: dW4t = dZ^T H3 ; db4 = colsum(dZ) ; dA3 = (dZ W4t) * (H3 > 0)
-  {
-    GemmArgs g = gemm_args(p->dZ, 1, kMlpOut, H[2], kMlpHid, 1, kMlpOut, kMlpHid, (int)n);
-    g.Cf = p->g + mlp_weight_offset(3);
-    g.scm = kMlpHid;
-    g.scn = 1;
-    gemm(ctx, s, g, "mlp_gemm_bwd", p);
-    colsum(ctx, s, p->dZ, (int)n, kMlpOut, kMlpOut, p->g + mlp_bias_offset(3), p);
-    GemmArgs h = gemm_args(p->dZ, kMlpOut, 1, mlp_wbf(p, 3), kMlpHid, 1, (int)n, kMlpHid, kMlpOut);
-    h.Cb = p->dA + 2 * B * kMlpHid;
-    h.scm = kMlpHid;
-    h.scn = 1;
-    h.mask = H[2];
-    h.smm = kMlpHid;
-    h.smn = 1;
-    gemm(ctx, s, h, "mlp_gemm_bwd", p);
-  }
-  for (int layer = 2; layer >= 0; --layer) {
-    const uint16_t *dA = p->dA + (size_t)layer * B * kMlpHid;
-    const uint16_t *in = layer == 0 ? p->X : H[layer - 1];
-    const int K = kMlpInPad;  // all hidden-layer inputs are 128 wide
-    GemmArgs g = gemm_args(dA, 1, kMlpHid, in, K, 1, kMlpHid, K, (int)n);
-    g.Cf = p->g + mlp_weight_offset(layer);
-    g.scm = K;
-    g.scn = 1;
-    gemm(ctx, s, g, "mlp_gemm_bwd", p);
-    colsum(ctx, s, dA, (int)n, kMlpHid, kMlpHid, p->g + mlp_bias_offset(layer), p);
-    if (layer > 0) {
-      GemmArgs h = gemm_args(dA, kMlpHid, 1, mlp_wbf(p, layer), kMlpInPad, 1, (int)n, kMlpHid, kMlpHid);
-      h.Cb = p->dA + (size_t)(layer - 1) * B * kMlpHid;
-      h.scm = kMlpHid;
-      h.scn = 1;
-      h.mask = H[layer - 1];
-      h.smm = kMlpHid;
-      h.smn = 1;
-      gemm(ctx, s, h, "mlp_gemm_bwd", p);
-    }
-  }
-}
-
-void mlp_adam(Context *ctx, hipStream_t s, Proposal *p, float lr) {
-  p->step += 1;
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  const float c1 = 1.f - std::pow(b1, (float)p->step), c2 = 1.f - std::pow(b2, (float)p->step);
-  launch(ctx, s, "mlp_adam", k_adam, dim3(blocks_for(kMlpParams, 256)), dim3(256), 0, p->w, (const float *)p->g, p->m,
-         p->v, (uint32_t)kMlpParams, lr, b1, b2, eps, c1, c2, (const uint32_t *)p->bfMap, p->wbf);
-  mlp_refresh_bias(ctx, s, p);
 }
 
 void mlp_labels_of_leaves(Context *ctx, hipStream_t s, Proposal *p, const int32_t *leaves, uint32_t n,
@@ -994,7 +556,7 @@ void mlp_infer(Context *ctx, hipStream_t s, Proposal *p, const void *rays, uint3
   const uint32_t classes = p->numClasses ? p->numClasses : (uint32_t)kMlpOut;
   const size_t ldsOut = 2 * 128 * 256 + (size_t)kMlpOut * 4;  // W4t ring + output bias
   launch(ctx, s, "mlp_infer_fused", k_infer_top1, dim3(blocks_for(n, kInferRays)), dim3(256), ldsOut, n,
-         mlp_wbf(p, 3), (const float *)p->bias, cls, logit, classes, gate,
+         mlp_wbf(p, 3), (const float *)p->weights.bias, cls, logit, classes, gate,
          (const GPRTRay *)rays, mlp_wbf(p, 0), mlp_wbf(p, 1), mlp_wbf(p, 2));
 }
 

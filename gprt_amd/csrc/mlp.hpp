@@ -27,22 +27,30 @@ constexpr size_t kMlpBiases = 3 * kMlpHid + kMlpOut;  // contiguous bias vector 
 inline size_t mlp_weight_offset(int layer) { return (size_t)layer * (kMlpW + kMlpHid); }
 inline size_t mlp_bias_offset(int layer) { return layer < 3 ? mlp_weight_offset(layer) + kMlpW : 3 * (kMlpW + kMlpHid) + kMlpW4; }
 inline size_t mlp_weight_size(int layer) { return layer < 3 ? kMlpW : kMlpW4; }
-inline size_t mlp_bf16_offset(int layer) { return (size_t)layer * kMlpW; }
+constexpr size_t mlp_bf16_offset(int layer) { return (size_t)layer * kMlpW; }
+
+// The bf16 weights in the layouts of their readers, and the biases b1 b2 b3 b4 in fp32.
+struct MlpWeights {
+  uint16_t *rows;  // W1t W2t W3t W4t, Wt[out][in]
+  uint16_t *fwd;   // MFMA fragments of W^T (mlp_train.hip)
+  uint16_t *bwd;   // MFMA fragments of W (W1's unused)
+  float *bias;
+};
 
 struct Proposal {
   void *block = nullptr;
   size_t blockBytes = 0;
   uint32_t maxBatch = 0;
   float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // fp32 params, grads, Adam moments
-  uint32_t *bfMap = nullptr;   // flat param index -> bf16 weight index (or ~0)
-  uint16_t *wbf = nullptr;     // bf16 weights W1t W2t W3t W4t
-  float *bias = nullptr;       // b1 b2 b3 b4 contiguous
+  MlpWeights weights{};
   float *stats = nullptr;      // [0] loss sum, [1] correct count (as uint)
-  uint16_t *X = nullptr, *H = nullptr, *dA = nullptr, *dZ = nullptr;
-  float *Z = nullptr;
-  int32_t *labels = nullptr;
-  float *gemmWs = nullptr;  // split-K partial sums of the training GEMMs
-  size_t gemmWsBytes = 0;
+  uint16_t *X = nullptr, *H = nullptr;  // features and hidden activations of gprtProposalLogits
+  float *Z = nullptr;                   // its logits
+  // A training batch: activations and their gradients, dZ (bf16 fragments), and the products' partial
+  // sums (mlp_train_bytes).
+  uint16_t *act = nullptr, *dZ = nullptr;
+  float *trainWs = nullptr;
+  float *rowLoss = nullptr;
   uint32_t step = 0;
   // Treelets of the accel the proposal serves.
   void *treeBlock = nullptr;
@@ -69,10 +77,20 @@ size_t mlp_param_count();
 bool mlp_alloc(Context *ctx, Proposal *p, uint32_t maxBatch);
 void mlp_release(Proposal *p);
 bool mlp_set_params(Context *ctx, hipStream_t s, Proposal *p, const float *host);
-bool mlp_refresh_bias(Context *ctx, hipStream_t s, Proposal *p);
+// Writes the bf16 weights and the biases from the fp32 parameters.
+void mlp_store_params(Context *ctx, hipStream_t s, Proposal *p);
 void mlp_forward_batch(Context *ctx, hipStream_t s, Proposal *p, const void *rays, uint32_t n);
-void mlp_backward_batch(Context *ctx, hipStream_t s, Proposal *p, uint32_t n, uint32_t labelled);
-void mlp_adam(Context *ctx, hipStream_t s, Proposal *p, float lr);
+// One minibatch of n <= maxBatch rays: forward, backward and Adam; loss (mean over the batch) and top-1
+// count are added to stats.
+void mlp_train_step(Context *ctx, hipStream_t s, Proposal *p, const void *rays, const int32_t *labels, uint32_t n,
+                    float lr);
+// The gradient of the mean cross-entropy over `labelled` rays, into p->g.
+void mlp_gradients(Context *ctx, hipStream_t s, Proposal *p, const void *rays, const int32_t *labels, uint32_t n,
+                   uint32_t labelled);
+struct TrainBytes {
+  size_t act, dz, loss, ws;
+};
+TrainBytes mlp_train_bytes(uint32_t maxBatch);
 void mlp_labels(Context *ctx, hipStream_t s, Proposal *p, const void *hits, uint32_t n, int32_t *labels);
 // Classes of top-level leaves (instance accels): labels[i] = leafClass[leaves[i]], or -1.
 void mlp_labels_of_leaves(Context *ctx, hipStream_t s, Proposal *p, const int32_t *leaves, uint32_t n,

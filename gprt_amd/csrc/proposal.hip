@@ -338,10 +338,8 @@ GPRT_API void gprtProposalGradients(GPRTContext _ctx, GPRTProposal _p, GPRTBuffe
     return;
   }
   hipStream_t s = ctx->stream;
-  hip_ok(hipMemcpyAsync(p->labels, labels->d, (size_t)count * 4, hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
   fill_u32(ctx, s, p->stats, 0u, 2);
-  mlp_forward_batch(ctx, s, p, rays->d, count);
-  mlp_backward_batch(ctx, s, p, count, count);
+  mlp_gradients(ctx, s, p, rays->d, (const int32_t *)labels->d, count, count);
   hip_ok(hipMemcpyAsync(hostGrads, p->g, kMlpParams * 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(grads)");
   hipStreamSynchronize(s);
 }
@@ -386,10 +384,7 @@ float train_core(Context *ctx, Proposal *p, const void *rays, const void *hits, 
     uint32_t batches = 0;
     for (uint32_t b0 = 0; b0 < labelled; b0 += p->maxBatch) {
       const uint32_t n = std::min<uint32_t>(p->maxBatch, labelled - b0);
-      hip_ok(hipMemcpyAsync(p->labels, cLabels + b0, (size_t)n * 4, hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
-      mlp_forward_batch(ctx, s, p, cRays + b0, n);
-      mlp_backward_batch(ctx, s, p, n, n);
-      mlp_adam(ctx, s, p, lr);
+      mlp_train_step(ctx, s, p, cRays + b0, cLabels + b0, n, lr);
       ++batches;
     }
     float st[2];

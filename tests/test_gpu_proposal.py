@@ -163,6 +163,40 @@ def test_gradients_match_cpu(ctx):
     prop.destroy()
 
 
+# Around the 16 rays of a workgroup, the 32 of a product's step, the 256 of a bias sum and the sizes at which
+# the products split, in a batch that is not a multiple of any; the bounds are those above.
+@pytest.mark.parametrize("n", [1, 16, 17, 33, 255, 257, 511, 513, 1100])
+def test_gradients_at_ragged_sizes(ctx, n):
+    prop = api.Proposal(ctx, max_batch=1111, seed=1)
+    p = M.he_init(n).astype(np.float32)
+    prop.set_params(p)
+    rays = scenes.random_rays(n, seed=n)
+    labels = np.random.default_rng(n).integers(0, 4096, n).astype(np.int32)
+    rb, lb = ctx.device_buffer(rays), ctx.device_buffer(labels)
+    g = np.full(prop.n_params, np.nan, dtype=np.float32)
+    ctx.lib.gprtProposalGradients(ctx.h, prop.h, rb.h, lb.h, n, g.ctypes.data_as(C.c_void_p), len(g))
+    assert api.last_error() is None, api.last_error()
+    _, ref = M.loss_and_grad(p.astype(np.float64), M.encode(rays), labels, bf16=True, bf16_grads=True)
+    for layer, (w0, shape, b0, bn) in enumerate(M.offsets()):
+        for name, sl in ((f"W{layer + 1}", slice(w0, w0 + shape[0] * shape[1])), (f"b{layer + 1}", slice(b0, b0 + bn))):
+            assert _relnorm(g[sl], ref[sl]) <= NORM_TOL, name
+    # Unlabelled rays add nothing: which rays they are does not matter.
+    labels[::2] = -1
+    lb.write(labels)
+    some = []
+    for seed in (n, n + 1):
+        rays[::2] = scenes.random_rays(n, seed=seed)[::2]
+        rb.write(rays)
+        h = np.full(prop.n_params, np.nan, dtype=np.float32)
+        ctx.lib.gprtProposalGradients(ctx.h, prop.h, rb.h, lb.h, n, h.ctypes.data_as(C.c_void_p), len(h))
+        some.append(h)
+    np.testing.assert_array_equal(some[0], some[1])
+    assert np.any(some[0]) == (n > 1)
+    rb.destroy()
+    lb.destroy()
+    prop.destroy()
+
+
 def test_treelet_cut(ctx, scene):
     verts, idx, acc = scene
     prop = api.Proposal(ctx, max_batch=256, seed=1)
