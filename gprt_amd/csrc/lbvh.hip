@@ -879,11 +879,18 @@ __global__ void __launch_bounds__(kBuildSub) k_build_sub(BuildArgs a, uint32_t t
 //
 // A level's input is the outputs of the level below, in leaf order: subtrees that partition its
 // range, each with its box, its reference (inner index or ~leaf), its first leaf L and delta(L-1).
-// Treating each subtree as one leaf, the same rule builds the nodes above them: with D[i] =
-// delta(L_i - 1) and D[S] the delta after the range, the node over subtrees [a, b] goes to the
-// boundary after b when D[b+1] > D[a] (a left child), else to the boundary before a. Merges run
-// in rounds in LDS as in the sub-tile; nodes whose parent lies outside the window, and nodes still
-// waiting for a sibling at the end, are the window's outputs, again in leaf order.
+// Treating each subtree as one leaf, the same rule gives the nodes above them: with D[i] =
+// delta(L_i - 1) and D[S] the delta after the range, the node split at boundary g (between subtrees g
+// and g + 1) reaches left to the nearest a <= g with D[a] < D[g + 1] and right to the b before the
+// nearest j >= g + 2 with D[j] < D[g + 1]. (Between two boundaries of equal delta there is always one of
+// a smaller: the one that separates their prefixes.) A node whose a or j lies beyond the window is not
+// finished there; the subtrees and finished nodes without a finished parent are the window's outputs,
+// again in leaf order.
+//
+// All nodes are found at once rather than by merge rounds, which are a chain of as many LDS round trips
+// as the tree has levels (about 0.76 us each): the reaches by descending a table of minima of D over
+// powers of two, the boxes as the union of two overlapping powers of two of the input boxes, one
+// barrier per power.
 //
 // A window holds at most kMergeCap subtrees. A longer sequence is merged window by window, the
 // outputs of each window replacing its inputs at the front of the same list, until one window
@@ -893,164 +900,223 @@ __global__ void __launch_bounds__(kBuildSub) k_build_sub(BuildArgs a, uint32_t t
 // at most 130 entries), and its outputs are at most 2 x 65 subtrees (one per tree level on each
 // side).
 // ------------------------------------------------------------------------------------------------
-// Regions: windows of 1024 subtrees (512 threads, 75 KB of LDS: two workgroups per CU). The top
-// level runs one workgroup per large mesh and takes windows of 2048 (1024 threads, 150 KB), so a
-// mesh of up to ~128 regions merges in one window.
+// Regions: windows of 1024 subtrees (one per thread, 69 KB of LDS: two workgroups per CU). The top level
+// runs one workgroup per large mesh and takes windows of 2048 (two per thread, 145 KB), so a mesh of up
+// to ~128 regions merges in one window.
 constexpr uint32_t kRegionCap = 1024, kTopCap = 2048;
+constexpr int kMergeThreads = 1024;
 
-template <uint32_t kMergeCap>
-struct MergeLds {
-  static constexpr int kMergeThreads = kMergeCap / 2;  // the output pass takes two subtrees per thread
-  float leafBox[kMergeCap][6];   // input subtrees' boxes
-  float nodeBox[kMergeCap][6];   // merged nodes' boxes, by boundary
-  int ref[kMergeCap];            // input subtrees' references
-  uint32_t node[kMergeCap];      // merged nodes' inner indices, by boundary
-  uint32_t L[kMergeCap + 1];     // first leaf of each input subtree; [S]: the position after the window
-  int8_t D[kMergeCap + 4];       // delta(L - 1) of each input subtree; [S]: the delta after the window
-  uint32_t meet[kMergeCap / 4];  // sides arrived per boundary, 8 bits each
-  uint16_t child[kMergeCap][2];  // the arrived child per side: local id (< kMergeCap input, else node)
-  uint16_t far[kMergeCap][2];    // its far input subtree (first of a left child, last of a right child)
-  uint16_t ready[2][kMergeCap / 2];
-  uint16_t out[kMergeCap];       // local id of the output starting at each input subtree (0xFFFF: none)
-  uint32_t nready[3];
-  uint32_t wsum[kMergeThreads / 64 + 1];
+// A box as order-preserving integers, which min / max leave exact: {lo.x lo.y} {lo.z hi.x} {hi.y hi.z}.
+struct OrdBox {
+  uint2 a, b, c;
+};
+__device__ __forceinline__ OrdBox ord_box(const float b[6]) {
+  return {make_uint2(ford(b[0]), ford(b[1])), make_uint2(ford(b[2]), ford(b[3])), make_uint2(ford(b[4]), ford(b[5]))};
+}
+__device__ __forceinline__ void float_box(const OrdBox &o, float b[6]) {
+  const uint32_t u[6] = {o.a.x, o.a.y, o.b.x, o.b.y, o.c.x, o.c.y};
+#pragma unroll
+  for (int c = 0; c < 6; ++c) b[c] = unord(u[c]);
+}
+__device__ __forceinline__ OrdBox join(const OrdBox &x, const OrdBox &y) {
+  return {make_uint2(min(x.a.x, y.a.x), min(x.a.y, y.a.y)), make_uint2(min(x.b.x, y.b.x), max(x.b.y, y.b.y)),
+          make_uint2(max(x.c.x, y.c.x), max(x.c.y, y.c.y))};
+}
+
+// Tables over a sequence of up to kCap subtrees: boxes of the power of two at hand (two of them, written
+// in turn), and minima of D over every power of two.
+template <uint32_t kCap>
+struct RangeTables {
+  static constexpr int kLevels = kCap == 1024 ? 11 : 12;  // 2^(kLevels - 1) = kCap
+  static_assert(kCap == 1024 || kCap == 2048, "kLevels");
+  uint2 box[2][3][kCap];
+  int8_t D[kLevels][kCap + 8];  // D[k][i] = min of D[0][i .. i + 2^k)
+
+  __device__ __forceinline__ OrdBox get(int buf, uint32_t i) const { return {box[buf][0][i], box[buf][1][i], box[buf][2][i]}; }
+  __device__ __forceinline__ void put(int buf, uint32_t i, const OrdBox &o) {
+    box[buf][0][i] = o.a;
+    box[buf][1][i] = o.b;
+    box[buf][2][i] = o.c;
+  }
 };
 
-// Merges input subtrees [0, S) (already in LDS: leafBox, ref, L[0..S], D[0..S]) and appends the
-// window's outputs at out[*outCount...] (outD: their deltas). Called by every thread.
-template <uint32_t kMergeCap>
-__device__ void merge_window(MergeLds<kMergeCap> &sm, uint32_t S, uint32_t n, BVHNode *__restrict__ nodes, float *__restrict__ header,
-                             Subtree *__restrict__ out, int8_t *__restrict__ outD, uint32_t outBase,
-                             uint32_t &outCount) {
-  constexpr int kMergeThreads = MergeLds<kMergeCap>::kMergeThreads;
+// Fills the minima over D[0][0 .. S]; returns the largest power's exponent. Called by every thread, after a
+// barrier that orders D[0]; ends with one.
+template <uint32_t kCap>
+__device__ __forceinline__ int minima(RangeTables<kCap> &t, uint32_t S) {
+  int k = 0;
+  for (; (2u << k) <= S + 1u; ++k) {
+    for (uint32_t i = threadIdx.x; i + (2u << k) <= S + 1u; i += kMergeThreads)
+      t.D[k + 1][i] = min(t.D[k][i], t.D[k][i + (1u << k)]);
+    lds_barrier();
+  }
+  return k;
+}
+
+// The reach [a, b] of the node split at boundary g; false if it leaves the sequence.
+template <uint32_t kCap>
+__device__ __forceinline__ bool reach(const RangeTables<kCap> &t, uint32_t S, int top, uint32_t g, uint32_t &a, uint32_t &b) {
+  const int d = t.D[0][g + 1];
+  int left = (int)g;
+  uint32_t right = g + 2u;
+  for (int k = top; k >= 0; --k) {
+    const uint32_t w = 1u << k;
+    if (left + 1 >= (int)w && t.D[k][left + 1 - (int)w] >= d) left -= (int)w;
+    if (right + w <= S + 1u && t.D[k][right] >= d) right += w;
+  }
+  a = (uint32_t)left;
+  b = right - 1u;
+  return left >= 0 && right <= S;
+}
+
+// Karras index of the node over leaves [pl, pr] with deltas dl before and dr after it.
+__device__ __forceinline__ uint32_t karras_index(int dl, int dr, uint32_t pl, uint32_t pr) {
+  return (dl < 0 && dr < 0) ? 0u : (dr > dl ? pr : pl);
+}
+
+template <uint32_t kCap>
+struct MergeLds {
+  RangeTables<kCap> t;
+  int ref[kCap];             // input subtrees' references
+  uint32_t L[kCap + 1];      // first leaf of each input subtree; [S]: the position after the window
+  uint32_t fin[kCap / 32];   // boundaries whose node is finished in the window
+  uint32_t outs[kCap / 32];  // input subtrees at which an output starts
+  uint32_t rank[kCap / 32 + 1];
+};
+
+// Merges input subtrees [0, S) (already in LDS: boxes, ref, L[0..S], D[0..S]) and appends the
+// window's outputs at out[outBase + *outCount...] (outD: their deltas). Called by every thread.
+template <uint32_t kCap>
+__device__ void merge_window(MergeLds<kCap> &sm, uint32_t S, uint32_t n, BVHNode *__restrict__ nodes,
+                             float *__restrict__ header, Subtree *__restrict__ out, int8_t *__restrict__ outD,
+                             uint32_t outBase, uint32_t &outCount) {
+  constexpr uint32_t kPer = kCap / kMergeThreads;  // thread tid takes subtrees and boundaries tid + t * threads
   const uint32_t tid = threadIdx.x;
-  auto box_of = [&](uint32_t id) -> const float * { return id < kMergeCap ? sm.leafBox[id] : sm.nodeBox[id - kMergeCap]; };
-  auto ref_of = [&](uint32_t id) -> int { return id < kMergeCap ? sm.ref[id] : (int)sm.node[id - kMergeCap]; };
-  // The node over input subtrees [fa, fb] (local id `id`, box in LDS) arrives at its parent's
-  // boundary.
-  auto arrive = [&](uint32_t fa, uint32_t fb, uint32_t id, uint32_t nextQ) {
-    const int dl = sm.D[fa], dr = sm.D[fb + 1];
-    if (dl < 0 && dr < 0) {  // the whole mesh: the root
-      const float *b = box_of(id);
-      for (int c = 0; c < 6; ++c) header[8 + c] = b[c];
-      return;
-    }
-    const bool leftChild = dr > dl;
-    if (leftChild ? fb + 1u >= S : fa == 0u) {  // the parent lies outside the window
-      sm.out[fa] = (uint16_t)id;
-      return;
-    }
-    const uint32_t g = leftChild ? fb : fa - 1u, side = leftChild ? 0u : 1u;
-    sm.child[g][side] = (uint16_t)id;
-    sm.far[g][side] = (uint16_t)(leftChild ? fa : fb);
-    const uint32_t shift = (g & 3u) * 8u;
-    const uint32_t old = __hip_atomic_fetch_or(&sm.meet[g >> 2], (1u << side) << shift, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-    if ((old >> shift) & 3u) {
-      const uint32_t slot =
-          __hip_atomic_fetch_add(&sm.nready[nextQ % 3], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      sm.ready[nextQ & 1][slot] = (uint16_t)g;
-    }
-  };
-  for (uint32_t i = tid; i < kMergeCap / 4; i += kMergeThreads) sm.meet[i] = 0u;
-  for (uint32_t i = tid; i < S; i += kMergeThreads) sm.out[i] = 0xFFFFu;
-  if (tid < 3) sm.nready[tid] = 0u;
-  lds_barrier();
-  for (uint32_t i = tid; i < S; i += kMergeThreads) arrive(i, i, i, 1u);
-  lds_barrier();
-  for (uint32_t round = 1; round <= kMergeCap; ++round) {
-    const uint32_t count = sm.nready[round % 3];
-    if (count == 0u) break;  // uniform: read after the barrier
-    if (tid == 0) sm.nready[(round + 2) % 3] = 0u;
-    for (uint32_t q = tid; q < count; q += kMergeThreads) {
-      const uint32_t g = sm.ready[round & 1][q];
-      const uint32_t i0 = sm.child[g][0], i1 = sm.child[g][1];
-      const uint32_t fa = sm.far[g][0], fb = sm.far[g][1];
-      const uint32_t pl = sm.L[fa], pr = sm.L[fb + 1] - 1u;
-      const int pdl = sm.D[fa], pdr = sm.D[fb + 1];
-      const uint32_t P = (pdl < 0 && pdr < 0) ? 0u : (pdr > pdl ? pr : pl);
-      const float *p0 = box_of(i0), *p1 = box_of(i1);
-      float b0[6], b1[6];
-      for (int c = 0; c < 6; ++c) {
-        b0[c] = p0[c];
-        b1[c] = p1[c];
+  auto &tb = sm.t;
+  for (uint32_t i = tid; i < kCap / 32; i += kMergeThreads) sm.fin[i] = sm.outs[i] = 0u;
+  const int top = minima(tb, S);
+  uint32_t a[kPer], b[kPer];
+  bool fin[kPer];
+#pragma unroll
+  for (uint32_t t = 0; t < kPer; ++t) {
+    const uint32_t g = tid + t * kMergeThreads;
+    fin[t] = g + 1u < S && reach(tb, S, top, g, a[t], b[t]);
+    if (fin[t]) atomicOr(&sm.fin[g >> 5], 1u << (g & 31u));
+  }
+  // Boxes: the input's own, and of the finished node's two children [a, g] and [g + 1, b].
+  OrdBox own[kPer], c0[kPer], c1[kPer];
+#pragma unroll
+  for (uint32_t t = 0; t < kPer; ++t) own[t] = tb.get(0, tid + t * kMergeThreads);
+  for (int k = 0; (1u << k) <= S; ++k) {
+    const int buf = k & 1;
+    const uint32_t w = 1u << k;
+#pragma unroll
+    for (uint32_t t = 0; t < kPer; ++t) {
+      const uint32_t g = tid + t * kMergeThreads;
+      if (fin[t]) {
+        const uint32_t n0 = g - a[t] + 1u, n1 = b[t] - g;
+        if (n0 >> k == 1u) c0[t] = join(tb.get(buf, a[t]), tb.get(buf, g + 1u - w));
+        if (n1 >> k == 1u) c1[t] = join(tb.get(buf, g + 1u), tb.get(buf, b[t] + 1u - w));
       }
-      if (P + 1u < n) write_node(&nodes[P], b0, b1, ref_of(i0), ref_of(i1), P == pl ? pr : pl);
-      merge_box(b0, b1);
-      for (int c = 0; c < 6; ++c) sm.nodeBox[g][c] = b0[c];
-      sm.node[g] = P;
-      arrive(fa, fb, kMergeCap + g, round + 1u);
+    }
+    if (2u * w > S) break;
+#pragma unroll
+    for (uint32_t t = 0; t < kPer; ++t) {
+      const uint32_t i = tid + t * kMergeThreads;
+      if (i + 2u * w <= S) tb.put(buf ^ 1, i, join(tb.get(buf, i), tb.get(buf, i + w)));
     }
     lds_barrier();
   }
-  // Boundaries with one child arrived: its sibling lies partly outside the window.
-  for (uint32_t g = tid; g + 1u < S; g += kMergeThreads) {
-    const uint32_t meet = (sm.meet[g >> 2] >> ((g & 3u) * 8u)) & 3u;
-    if (meet == 1u || meet == 2u) {
-      const uint32_t side = meet >> 1;
-      sm.out[side == 0 ? sm.far[g][0] : g + 1u] = sm.child[g][side];
+  if (S == 1u) lds_barrier();  // otherwise a level's barrier has ordered sm.fin
+  // The node over [fa, fb] is an output when its parent's boundary lies outside or is not finished; the
+  // root is none.
+  auto is_output = [&](uint32_t fa, uint32_t fb) {
+    const int dl = tb.D[0][fa], dr = tb.D[0][fb + 1];
+    if (dl < 0 && dr < 0) return false;
+    const bool leftChild = dr > dl;
+    if (leftChild ? fb + 1u >= S : fa == 0u) return true;
+    const uint32_t g = leftChild ? fb : fa - 1u;
+    return !(sm.fin[g >> 5] >> (g & 31u) & 1u);
+  };
+  bool outIn[kPer], outNode[kPer];
+#pragma unroll
+  for (uint32_t t = 0; t < kPer; ++t) {
+    const uint32_t i = tid + t * kMergeThreads;
+    outIn[t] = i < S && is_output(i, i);
+    outNode[t] = fin[t] && is_output(a[t], b[t]);
+    if (outIn[t]) atomicOr(&sm.outs[i >> 5], 1u << (i & 31u));
+    if (outNode[t]) atomicOr(&sm.outs[a[t] >> 5], 1u << (a[t] & 31u));
+    if (i < S && tb.D[0][i] < 0 && tb.D[0][i + 1] < 0) {  // one subtree is the whole mesh
+      float bx[6];
+      float_box(own[t], bx);
+      for (int c = 0; c < 6; ++c) header[8 + c] = bx[c];
+    }
+    if (fin[t]) {
+      const uint32_t g = i, pl = sm.L[a[t]], pr = sm.L[b[t] + 1u] - 1u, mid = sm.L[g + 1u];
+      const int dl = tb.D[0][a[t]], dr = tb.D[0][b[t] + 1u];
+      const uint32_t P = karras_index(dl, dr, pl, pr);
+      float b0[6], b1[6];
+      float_box(c0[t], b0);
+      float_box(c1[t], b1);
+      // A left child's index is its last leaf, a right child's its first.
+      const int r0 = a[t] == g ? sm.ref[g] : (int)(mid - 1u), r1 = b[t] == g + 1u ? sm.ref[g + 1u] : (int)mid;
+      if (P + 1u < n) write_node(&nodes[P], b0, b1, r0, r1, P == pl ? pr : pl);
+      if (dl < 0 && dr < 0) {
+        merge_box(b0, b1);
+        for (int c = 0; c < 6; ++c) header[8 + c] = b0[c];
+      }
     }
   }
   lds_barrier();
-  // Outputs in leaf order: thread t takes input subtrees [2t, 2t + 1].
-  const uint32_t i0 = 2 * tid, i1 = 2 * tid + 1;
-  const bool o0 = i0 < S && sm.out[i0] != 0xFFFFu, o1 = i1 < S && sm.out[i1] != 0xFFFFu;
-  const uint32_t mine = (uint32_t)o0 + (uint32_t)o1;
-  const uint32_t lane = tid & 63u, wave = tid >> 6;
-  const uint32_t incl = wave_incl_sum(mine);
-  if (lane == 63u) sm.wsum[wave] = incl;
-  lds_barrier();
-  if (tid == 0) {
-    uint32_t run = 0;
-    for (uint32_t w = 0; w < kMergeThreads / 64; ++w) {
-      const uint32_t c = sm.wsum[w];
-      sm.wsum[w] = run;
-      run += c;
-    }
-    sm.wsum[kMergeThreads / 64] = run;
+  constexpr uint32_t kWords = kCap / 32;
+  if (tid < 64) {
+    const uint32_t c = tid < kWords ? (uint32_t)__popc(sm.outs[tid]) : 0u;
+    const uint32_t incl = wave_incl_sum(c);
+    if (tid < kWords) sm.rank[tid] = incl - c;
+    if (tid == kWords - 1) sm.rank[kWords] = incl;
   }
+  static_assert(kWords <= 64, "one wave ranks the outputs");
   lds_barrier();
-  uint32_t rank = outBase + outCount + sm.wsum[wave] + incl - mine;
-  for (uint32_t j = 0; j < 2; ++j) {
-    const uint32_t i = i0 + j;
-    if (!(j == 0 ? o0 : o1)) continue;
-    const uint32_t id = sm.out[i];
-    const float *pb = box_of(id);
-    float b[6];
-    for (int c = 0; c < 6; ++c) b[c] = pb[c];
-    put_entry(&out[rank], b, ref_of(id), sm.L[i]);
-    outD[rank] = sm.D[i];
-    ++rank;
+  auto put = [&](uint32_t i, const OrdBox &o, int ref) {
+    const uint32_t r = outBase + outCount + sm.rank[i >> 5] + (uint32_t)__popc(sm.outs[i >> 5] & ((1u << (i & 31u)) - 1u));
+    float bx[6];
+    float_box(o, bx);
+    put_entry(&out[r], bx, ref, sm.L[i]);
+    outD[r] = tb.D[0][i];
+  };
+#pragma unroll
+  for (uint32_t t = 0; t < kPer; ++t) {
+    const uint32_t i = tid + t * kMergeThreads;
+    if (outIn[t]) put(i, own[t], sm.ref[i]);
+    if (outNode[t])
+      put(a[t], join(c0[t], c1[t]),
+          (int)karras_index(tb.D[0][a[t]], tb.D[0][b[t] + 1u], sm.L[a[t]], sm.L[b[t] + 1u] - 1u));
   }
-  outCount += sm.wsum[kMergeThreads / 64];
+  outCount += sm.rank[kWords];
   // The outputs may overwrite inputs of this list that the next window or pass loads.
   __syncthreads();
 }
 
 // Loads input subtrees [w0, w0 + S) of a sequence into LDS; `at(e)` gives entry e's index in
 // `in` / `inD`. endL / endD describe what follows the sequence when the window reaches its end.
-template <uint32_t kMergeCap, class At>
-__device__ void load_window(MergeLds<kMergeCap> &sm, const Subtree *__restrict__ in, const int8_t *__restrict__ inD, At at,
+template <uint32_t kCap, class At>
+__device__ void load_window(MergeLds<kCap> &sm, const Subtree *__restrict__ in, const int8_t *__restrict__ inD, At at,
                             uint32_t w0, uint32_t S, uint32_t total, uint32_t endL, int endD) {
-  for (uint32_t i = threadIdx.x; i <= S; i += MergeLds<kMergeCap>::kMergeThreads) {
+  for (uint32_t i = threadIdx.x; i <= S; i += kMergeThreads) {
     const uint32_t e = w0 + i;
     if (e < total) {
       const size_t x = at(e);
       const float4 p = in[x].a, q = in[x].b;
       sm.L[i] = __float_as_uint(q.w);
-      sm.D[i] = inD[x];
+      sm.t.D[0][i] = inD[x];
       if (i < S) {
-        sm.leafBox[i][0] = p.x;
-        sm.leafBox[i][1] = p.y;
-        sm.leafBox[i][2] = p.z;
-        sm.leafBox[i][3] = q.x;
-        sm.leafBox[i][4] = q.y;
-        sm.leafBox[i][5] = q.z;
+        const float bx[6] = {p.x, p.y, p.z, q.x, q.y, q.z};
+        sm.t.put(0, i, ord_box(bx));
         sm.ref[i] = __float_as_int(p.w);
       }
     } else {  // i == S at the end of the sequence
       sm.L[i] = endL;
-      sm.D[i] = (int8_t)endD;
+      sm.t.D[0][i] = (int8_t)endD;
     }
   }
   lds_barrier();
@@ -1058,19 +1124,20 @@ __device__ void load_window(MergeLds<kMergeCap> &sm, const Subtree *__restrict__
 
 // Merges a whole sequence of `total` input subtrees: window by window (outputs compacted into
 // `tmp` / `tmpD` from its start) until one window holds what is left, whose outputs go to `dst`.
-// `at` maps entry e of the first pass to its index in `in`. Returns the number of outputs.
-template <uint32_t kMergeCap, class At>
-__device__ uint32_t merge_sequence(MergeLds<kMergeCap> &sm, const Subtree *in, const int8_t *inD, At at, uint32_t total,
+// `at` maps entry e of the first pass to its index in `in`; `tmp` may be the list that `in` is, if the
+// entries of the first pass are not before their index there. Returns the number of outputs.
+template <uint32_t kCap, class At>
+__device__ uint32_t merge_sequence(MergeLds<kCap> &sm, const Subtree *in, const int8_t *inD, At at, uint32_t total,
                                    uint32_t endL, int endD, Subtree *tmp, int8_t *tmpD, Subtree *dst, int8_t *dstD,
                                    uint32_t n, BVHNode *nodes, float *header) {
   bool first = true;
-  // Each pass leaves at most 130 outputs per window of kMergeCap, so passes end; the bound only
+  // Each pass leaves at most 130 outputs per window of kCap, so passes end; the bound only
   // guards against malformed keys.
   for (int pass = 0; pass < 16 && total > 0; ++pass) {
-    const bool last = total <= kMergeCap;
+    const bool last = total <= kCap;
     uint32_t outCount = 0;
-    for (uint32_t w0 = 0; w0 < total; w0 += kMergeCap) {
-      const uint32_t S = min(kMergeCap, total - w0);
+    for (uint32_t w0 = 0; w0 < total; w0 += kCap) {
+      const uint32_t S = min(kCap, total - w0);
       if (first) load_window(sm, in, inD, at, w0, S, total, endL, endD);
       else load_window(sm, tmp, tmpD, [](uint32_t e) { return (size_t)e; }, w0, S, total, endL, endD);
       merge_window(sm, S, n, nodes, header, last ? dst : tmp, last ? dstD : tmpD, 0u, outCount);
@@ -1082,9 +1149,20 @@ __device__ uint32_t merge_sequence(MergeLds<kMergeCap> &sm, const Subtree *in, c
   return 0u;
 }
 
+// Index j with pre[j] <= e < pre[j + 1], pre ascending over [0, count].
+__device__ __forceinline__ uint32_t list_of(const uint32_t *pre, uint32_t count, uint32_t e) {
+  uint32_t j = 0, jh = count;
+  while (jh - j > 1) {
+    const uint32_t mid = (j + jh) >> 1;
+    if (pre[mid] <= e) j = mid;
+    else jh = mid;
+  }
+  return j;
+}
+
 // Level 2: one workgroup per 65536-key region merges the outputs of its sub-tiles (each sub-tile's
 // list at its own key positions in list0) into list1 at the region's key positions.
-__global__ void __launch_bounds__(kRegionCap / 2) k_build_region(BuildArgs a, uint32_t regionBase) {
+__global__ void __launch_bounds__(kMergeThreads) __attribute__((amdgpu_waves_per_eu(8))) k_build_region(BuildArgs a, uint32_t regionBase) {
   __shared__ MergeLds<kRegionCap> sm;
   __shared__ uint32_t s_pre[kBuildRegion / kBuildSub + 1];
   const uint32_t t = a.regionTile[regionBase + blockIdx.x];  // the region's first tile
@@ -1117,12 +1195,7 @@ __global__ void __launch_bounds__(kRegionCap / 2) k_build_region(BuildArgs a, ui
   const uint32_t total = s_pre[nsub];
   const size_t base = (size_t)d.primOffset + regionLo;
   auto at = [&](uint32_t e) -> size_t {
-    uint32_t j = 0, jh = nsub;  // the sub-tile j with s_pre[j] <= e < s_pre[j + 1]
-    while (jh - j > 1) {
-      const uint32_t mid = (j + jh) >> 1;
-      if (s_pre[mid] <= e) j = mid;
-      else jh = mid;
-    }
+    const uint32_t j = list_of(s_pre, nsub, e);
     return base + (size_t)j * kBuildSub + (e - s_pre[j]);
   };
   const uint32_t outs = merge_sequence(sm, a.list0, a.listD0, at, total, regionHi, endD, a.list1 + base,
@@ -1131,11 +1204,12 @@ __global__ void __launch_bounds__(kRegionCap / 2) k_build_region(BuildArgs a, ui
   if (threadIdx.x == 0) a.regionCount[t] = outs;
 }
 
-// Level 3: one workgroup per mesh gathers its regions' outputs into list0 (from the mesh's start)
-// and merges them up to the root.
-__global__ void __launch_bounds__(kTopCap / 2) k_build_top(BuildArgs a, uint32_t fromList, uint32_t meshBase) {
-  constexpr int kMergeThreads = kTopCap / 2;
+// Level 3: one workgroup per mesh merges its regions' outputs (in list1 at the regions' key positions) up
+// to the root; a sequence of several windows goes through list0.
+__global__ void __launch_bounds__(kMergeThreads) k_build_top(BuildArgs a, uint32_t fromList, uint32_t meshBase) {
   __shared__ MergeLds<kTopCap> sm;
+  __shared__ uint32_t s_pre[kMergeThreads + 1];  // prefix of a chunk's region counts
+  __shared__ uint32_t s_wsum[kMergeThreads / 64 + 1];
   const uint32_t m = fromList ? a.bigMesh[blockIdx.x] : meshBase + blockIdx.x;
   const MeshDesc d = a.desc[m];
   const uint32_t n = d.ntri;
@@ -1144,44 +1218,44 @@ __global__ void __launch_bounds__(kTopCap / 2) k_build_top(BuildArgs a, uint32_t
   const uint32_t regions = (n + kBuildRegion - 1) / kBuildRegion;
   const size_t base = d.primOffset;
   uint32_t total = 0;
-  uint32_t *pre = sm.L;  // a chunk's region-count prefix (kMergeThreads + 1 words)
+  // Meshes of at most 1024 regions (67M primitives) are merged from list1 as it is; larger ones are
+  // gathered into list0 first.
+  const bool direct = regions <= (uint32_t)kMergeThreads;
   for (uint32_t r0 = 0; r0 < regions; r0 += kMergeThreads) {
     const uint32_t r = r0 + threadIdx.x;
     const uint32_t c = r < regions ? min(a.regionCount[d.tileOffset + r * perRegion], min(kBuildRegion, n - r * kBuildRegion)) : 0u;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t incl = wave_incl_sum(c);
-    if (lane == 63u) sm.wsum[wave] = incl;
+    if (lane == 63u) s_wsum[wave] = incl;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t run = 0;
-      for (uint32_t w = 0; w < kMergeThreads / 64; ++w) {
-        const uint32_t v = sm.wsum[w];
-        sm.wsum[w] = run;
-        run += v;
-      }
-      sm.wsum[kMergeThreads / 64] = run;
+    uint32_t off = 0, all = 0;
+    for (uint32_t w = 0; w < kMergeThreads / 64; ++w) {
+      const uint32_t v = s_wsum[w];
+      if (w < wave) off += v;
+      all += v;
     }
+    s_pre[threadIdx.x + 1] = off + incl;
+    if (threadIdx.x == 0) s_pre[0] = 0u;
     __syncthreads();
-    pre[threadIdx.x + 1] = sm.wsum[wave] + incl;
-    if (threadIdx.x == 0) pre[0] = 0u;
-    __syncthreads();
-    const uint32_t chunk = pre[kMergeThreads], nr = min(regions - r0, (uint32_t)kMergeThreads);
-    for (uint32_t e = threadIdx.x; e < chunk; e += kMergeThreads) {
-      uint32_t j = 0, jh = nr;
-      while (jh - j > 1) {
-        const uint32_t mid = (j + jh) >> 1;
-        if (pre[mid] <= e) j = mid;
-        else jh = mid;
+    if (!direct) {
+      const uint32_t nr = min(regions - r0, (uint32_t)kMergeThreads);
+      for (uint32_t e = threadIdx.x; e < all; e += kMergeThreads) {
+        const uint32_t j = list_of(s_pre, nr, e);
+        const size_t src = base + (size_t)(r0 + j) * kBuildRegion + (e - s_pre[j]);
+        const size_t dst = base + total + e;
+        a.list0[dst] = a.list1[src];
+        a.listD0[dst] = a.listD1[src];
       }
-      const size_t src = base + (size_t)(r0 + j) * kBuildRegion + (e - pre[j]);
-      const size_t dst = base + total + e;
-      a.list0[dst] = a.list1[src];
-      a.listD0[dst] = a.listD1[src];
     }
-    total += chunk;
+    total += all;
     __syncthreads();
   }
-  merge_sequence(sm, a.list0 + base, a.listD0 + base, [](uint32_t e) { return (size_t)e; }, total, n, -1,
+  auto at = [&](uint32_t e) -> size_t {
+    if (!direct) return e;
+    const uint32_t j = list_of(s_pre, regions, e);
+    return (size_t)j * kBuildRegion + (e - s_pre[j]);
+  };
+  merge_sequence(sm, (direct ? a.list1 : a.list0) + base, (direct ? a.listD1 : a.listD0) + base, at, total, n, -1,
                  a.list0 + base, a.listD0 + base, a.list0 + base, a.listD0 + base, n, a.nodes + d.innerOffset,
                  a.headers + (size_t)m * 16);
 }
@@ -1307,14 +1381,14 @@ void launch_refit(Context *ctx, hipStream_t s, BVHStore *st, const BuildArgs &a,
   launch(ctx, s, "lbvh_build_local", k_build_sub, dim3(tiles * subPerTile), dim3(kBuildSub), 0, a, tileBase,
          subPerTile, afterBounds ? 1u : 0u);
   const uint32_t r0 = st->regionFirst[meshBase], r1 = st->regionFirst[meshBase + meshes];
-  if (r1 > r0) launch(ctx, s, "lbvh_build_region", k_build_region, dim3(r1 - r0), dim3(kRegionCap / 2), 0, a, r0);
+  if (r1 > r0) launch(ctx, s, "lbvh_build_region", k_build_region, dim3(r1 - r0), dim3(kMergeThreads), 0, a, r0);
   if (meshes == st->meshes) {
     if (st->bigMeshes)
-      launch(ctx, s, "lbvh_build_top", k_build_top, dim3(st->bigMeshes), dim3(kTopCap / 2), 0, a, 1u, 0u);
+      launch(ctx, s, "lbvh_build_top", k_build_top, dim3(st->bigMeshes), dim3(kMergeThreads), 0, a, 1u, 0u);
   } else {
     for (uint32_t m = meshBase; m < meshBase + meshes; ++m)
       if (st->desc[m].ntri > kBuildRegion)
-        launch(ctx, s, "lbvh_build_top", k_build_top, dim3(1), dim3(kTopCap / 2), 0, a, 0u, m);
+        launch(ctx, s, "lbvh_build_top", k_build_top, dim3(1), dim3(kMergeThreads), 0, a, 0u, m);
   }
 }
 
