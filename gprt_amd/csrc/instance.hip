@@ -276,7 +276,7 @@ __global__ void __launch_bounds__(256) k_tlas_index(uint32_t *__restrict__ idx, 
 }
 
 // Object-space ray of instance `ti` (fixed operation order, FP32).
-__device__ __forceinline__ RayPre object_ray(const TlasInst &ti, const GPRTRay &ray) {
+__device__ __forceinline__ RayPre object_ray(const TlasInst &ti, const RayPre &ray) {
   const float *m = ti.inv;
   const float ox = ((m[0] * ray.ox + m[1] * ray.oy) + m[2] * ray.oz) + m[3];
   const float oy = ((m[4] * ray.ox + m[5] * ray.oy) + m[6] * ray.oz) + m[7];
@@ -319,9 +319,29 @@ __global__ void __launch_bounds__(256) k_tlas_tag(TriRecord *__restrict__ topTri
   topTris[pos] = r;
 }
 
-// kPlain: no proposal, no per-ray fetch counts and fewer than kSmallTreePrims top-level leaves
-// (the common trace: no skip compares or fetch counter, 32-bit node and record offsets).
-template <bool kCheck, bool kPlain>
+// Top-level leaf `pos`: one triangle of one instance (a copy of its record), intersected in the
+// instance's space.
+template <bool kCheck, bool kSmall>
+__device__ __forceinline__ void top_leaf(const RayPre &rw, const TriRecord *__restrict__ topTris, uint32_t leaves,
+                                         const TlasInst *__restrict__ insts, const BlasDesc *__restrict__ pool,
+                                         int pos, HitState &h) {
+  if ((uint32_t)pos >= leaves) return;
+  const TriRecord tr = kSmall ? at32(topTris, (uint32_t)pos) : topTris[pos];
+  const int code = __float_as_int(tr.v1.w);
+  if (code < 0) return;
+  const uint32_t inst = (uint32_t)code & kLeafInstMask;
+  const int k = (int)__float_as_uint(tr.v2.w);
+  if (kCheck && !blas_live(pool, insts[inst])) return;
+  if ((uint32_t)code & kLeafIdentity) {
+    intersect_record(rw, tr, inst, k, h);
+  } else {
+    const RayPre ro = object_ray(insts[inst], rw);
+    intersect_record(ro, tr, inst, k, h);
+  }
+}
+
+// The general form: with a proposal, per-ray fetch counts, or kSmallTreePrims top-level leaves and more.
+template <bool kCheck>
 __global__ void __launch_bounds__(kTraceBlock)
     k_trace_tlas(const BVHNode *__restrict__ topNodes, const TriRecord *__restrict__ topTris, uint32_t leaves,
                  const TlasInst *__restrict__ insts,
@@ -334,10 +354,10 @@ __global__ void __launch_bounds__(kTraceBlock)
   const uint32_t gtid = blockIdx.x * kTraceBlock + tid;
   const LaneStack st{s_stack, tid, spill + (size_t)gtid * (kMaxStack - kLdsStack)};
   const int l = tid & 63;
-  while (true) {
-    uint32_t base = 0;
-    if (l == 0) base = atomicAdd(work, 64u);
-    base = __shfl(base, 0, 64);
+  const bool more = count > gridDim.x * kTraceBlock;
+  bool first = true;
+  do {
+    const uint32_t base = next_rays(work, first);
     if (base >= count) break;
     const uint32_t ri = base + (uint32_t)l;
     if (ri < count) {
@@ -348,7 +368,7 @@ __global__ void __launch_bounds__(kTraceBlock)
       uint32_t visits = 0;
       // With a proposal: the proposed class (a subtree of one instance's own tree) first, whose hit
       // tightens t; then the top-level walk, which finds that hit again and records its leaf.
-      if (!kPlain && proposal) {
+      if (proposal) {
         const int32_t c = proposal[ri];
         if (c >= 0 && (uint32_t)c < numClasses) {
           const int2 cn = classNodes[c];
@@ -358,7 +378,7 @@ __global__ void __launch_bounds__(kTraceBlock)
               if (ti.flags & kInstIdentity) {
                 visits += traverse<kMaxStack>(rw, ti.nodes, ti.tris, ti.n, cn.y, h, st, 0, (uint32_t)cn.x, -1);
               } else {
-                const RayPre ro = object_ray(ti, ray);
+                const RayPre ro = object_ray(ti, rw);
                 visits += traverse<kMaxStack>(ro, ti.nodes, ti.tris, ti.n, cn.y, h, st, 0, (uint32_t)cn.x, -1);
               }
             }
@@ -366,24 +386,10 @@ __global__ void __launch_bounds__(kTraceBlock)
         }
       }
       auto topLeaf = [&](int pos, int) __attribute__((always_inline)) {
-                                  // A top-level leaf: one triangle of one instance (a copy of its
-                                  // record), intersected in the instance's space.
-                                  if ((uint32_t)pos >= leaves) return;
-                                  const TriRecord tr = kPlain ? at32(topTris, (uint32_t)pos) : topTris[pos];
-                                  const int code = __float_as_int(tr.v1.w);
-                                  if (code < 0) return;
-                                  const uint32_t inst = (uint32_t)code & kLeafInstMask;
-                                  const int k = (int)__float_as_uint(tr.v2.w);
-                                  if (kCheck && !blas_live(pool, insts[inst])) return;
-                                  if ((uint32_t)code & kLeafIdentity) {
-                                    intersect_record(rw, tr, inst, k, h);
-                                  } else {
-                                    const RayPre ro = object_ray(insts[inst], ray);
-                                    intersect_record(ro, tr, inst, k, h);
-                                  }
-                                };
-      visits += walk_batched<kMaxStack, decltype(topLeaf) &, kPlain>(rw, topNodes, leaves, leaves == 1 ? ~0 : 0, h,
-                                                                     st, 0, kNoSkip, topLeaf);
+        top_leaf<kCheck, false>(rw, topTris, leaves, insts, pool, pos, h);
+      };
+      visits += walk_batched<kMaxStack, decltype(topLeaf) &>(rw, topNodes, leaves, leaves == 1 ? ~0 : 0, h, st, 0,
+                                                             kNoSkip, topLeaf);
       GPRTHit o;
       o.t = h.prim >= 0 ? h.t : ray.tmax;
       o.primID = h.prim;
@@ -392,9 +398,41 @@ __global__ void __launch_bounds__(kTraceBlock)
       store_hit_stream(hits + ri, o);
       if (instOut) instOut[ri] = h.prim >= 0 ? (int32_t)h.inst : -1;
       if (leafOut) leafOut[ri] = h.prim >= 0 ? h.leaf : -1;
-      if (!kPlain && visitsOut) visitsOut[ri] = visits;
+      if (visitsOut) visitsOut[ri] = visits;
     }
-  }
+  } while (more);
+}
+
+// The plain trace. Of the 103 vector registers it would take, 20 waves per CU leave it 96.
+template <bool kCheck>
+__global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5)))
+    k_trace_tlas_stream(const BVHNode *__restrict__ topNodes, const TriRecord *__restrict__ topTris, uint32_t leaves,
+                        const TlasInst *__restrict__ insts, const BlasDesc *__restrict__ pool,
+                        const GPRTRay *__restrict__ rays, GPRTHit *__restrict__ hits, uint32_t count,
+                        uint32_t chunk, uint32_t *__restrict__ work, uint32_t *__restrict__ spill,
+                        int32_t *__restrict__ instOut, int32_t *__restrict__ leafOut) {
+  __shared__ StreamLds lds;
+  const uint32_t gtid = blockIdx.x * kTraceBlock + threadIdx.x;
+  RayPre rw = {};
+  SlabRay slab = {};
+  HitState h;
+  hit_init(h, 0.0f);
+  trace_stream(
+      topNodes, leaves, count, chunk, work, rw, slab, h, lds, spill + (size_t)gtid * (kMaxStack - kStreamStack),
+      [&](uint32_t ri) __attribute__((always_inline)) {
+        const GPRTRay ray = load_ray_stream(rays + ri);
+        rw = ray_setup(ray.ox, ray.oy, ray.oz, ray.tmin, ray.dx, ray.dy, ray.dz);
+        slab = slab_ray(rw);
+        hit_init(h, ray.tmax);
+      },
+      [&](int pos) __attribute__((always_inline)) {
+        top_leaf<kCheck, true>(rw, topTris, leaves, insts, pool, pos, h);
+      },
+      [&](uint32_t ri) __attribute__((always_inline)) {
+        store_hit_stream(hits + ri, GPRTHit{h.t, h.prim, h.u, h.v});  // t is still tmax if nothing was hit
+        if (instOut) instOut[ri] = h.prim >= 0 ? (int32_t)h.inst : -1;
+        if (leafOut) leafOut[ri] = h.prim >= 0 ? h.leaf : -1;
+      });
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -753,9 +791,6 @@ bool tlas_trace(Context *ctx, hipStream_t s, Accel *a, const void *rays, void *h
   Tlas *t = a->tlas;
   uint32_t *work = ensure_trace_scratch(ctx, s, kMaxStack - kLdsStack);
   if (!work) return false;
-  const unsigned blocks = (unsigned)ctx->cuCount * (blocksPerCU ? std::min<unsigned>(blocksPerCU, kBlocksPerCU)
-                                                               : (unsigned)kBlocksPerCU);
-  fill_u32(ctx, s, work, 0u, 1);
   // The proposal step walks the instances' own triangle accels, the top-level walk the copies
   // taken at this accel's build: once any triangle accel has changed since then, the proposal is
   // skipped so that hits stay those of the plain trace.
@@ -766,16 +801,28 @@ bool tlas_trace(Context *ctx, hipStream_t s, Accel *a, const void *rays, void *h
   const bool checked = t->builtEpoch != ctx->blasEpoch;
   const char *name = proposal ? "trace_closest_proposal_instances" : "trace_closest_instances";
   const bool plain = !proposal && !visits && t->leaves < kSmallTreePrims;
+  const TraceGrid g = trace_grid(ctx, count, plain, blocksPerCU);
+  if (g.counters) fill_u32(ctx, s, work, 0u, g.counters);
+  if (plain) {
+    auto go = [&](auto kernel) {
+      launch(ctx, s, name, kernel, dim3(g.blocks), dim3(kTraceBlock), 0, (const BVHNode *)t->top.nodes,
+             (const TriRecord *)t->top.tris, t->leaves, (const TlasInst *)t->insts, (const BlasDesc *)ctx->blasPool,
+             (const GPRTRay *)rays, (GPRTHit *)hits, count, g.chunk, work, work + kTraceHeaderWords,
+             instOut, leafOut);
+    };
+    checked ? go(k_trace_tlas_stream<true>) : go(k_trace_tlas_stream<false>);
+    return true;
+  }
   auto go = [&](auto kernel) {
-    launch(ctx, s, name, kernel, dim3(blocks), dim3(kTraceBlock), 0, (const BVHNode *)t->top.nodes,
+    launch(ctx, s, name, kernel, dim3(g.blocks), dim3(kTraceBlock), 0, (const BVHNode *)t->top.nodes,
            (const TriRecord *)t->top.tris, t->leaves, (const TlasInst *)t->insts, (const BlasDesc *)ctx->blasPool,
-           (const GPRTRay *)rays, (GPRTHit *)hits, count, work, work + 64, proposal, (const int2 *)t->classNodes, nc,
+           (const GPRTRay *)rays, (GPRTHit *)hits, count, work, work + kTraceHeaderWords, proposal, (const int2 *)t->classNodes, nc,
            instOut, leafOut, visits);
   };
   if (checked)
-    plain ? go(k_trace_tlas<true, true>) : go(k_trace_tlas<true, false>);
+    go(k_trace_tlas<true>);
   else
-    plain ? go(k_trace_tlas<false, true>) : go(k_trace_tlas<false, false>);
+    go(k_trace_tlas<false>);
   return true;
 }
 

@@ -300,7 +300,13 @@ bool sort_run(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAlt
 // Fill a device range with a 32-bit pattern (graph-safe; no hipMemset nodes).
 void fill_u32(Context *ctx, hipStream_t s, void *dst, uint32_t value, size_t words);
 
-// Trace work counter (first 256 B) + per-lane stack spill of `spillWordsPerLane` words.
+struct TraceGrid {
+  unsigned blocks;
+  uint32_t counters;  // words of the scratch's head to zero before the launch
+  uint32_t chunk;     // plain: rays a wave takes at a time
+};
+TraceGrid trace_grid(const Context *ctx, uint32_t count, bool plain, unsigned blocksPerCU);
+// Work counters (first kTraceHeaderWords words) + per-lane stack spill of `spillWordsPerLane` words.
 uint32_t *ensure_trace_scratch(Context *ctx, hipStream_t s, int spillWordsPerLane);
 
 // Triangle-accel descriptors (instance.hip).

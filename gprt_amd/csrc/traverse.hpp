@@ -1,11 +1,10 @@
 // Device-side closest-hit traversal shared by the triangle-accel and instance-accel trace kernels.
 //
-// One node fetch decides both children (64-byte node with both child boxes); leaf children are
-// handed to a leaf callback (at once by walk, in batches across the wave by walk_batched); the
-// near inner child is descended and the far one pushed on
-// a per-lane stack whose first kLdsStack entries live in LDS and the rest in a per-lane global
-// spill area. The stack is shared by nested traversals (instance accels: the bottom-level walk
-// starts above the top-level entries), so a traversal takes the stack slot it starts at.
+// One node fetch decides both children (64-byte node with both child boxes); leaf children are handed to
+// a leaf callback in batches across the wave; the near inner child is descended and the far one pushed on
+// a per-lane stack whose first entries live in LDS and the rest in a per-lane global spill area. A plain
+// trace runs trace_stream; with a proposal or fetch counts, or for trees of kSmallTreePrims primitives
+// and more, a lane walks one ray at a time with walk_batched.
 #pragma once
 
 #include <climits>
@@ -18,10 +17,26 @@ constexpr int kTraceBlock = 128;
 constexpr int kLdsStack = 20;
 // 14 workgroups (28 waves) per CU: 16, the most the LDS stacks allow, measured no faster.
 constexpr int kBlocksPerCU = 14;
-// A binary radix tree over distinct 64-bit keys is at most 64 levels deep, so a single-level walk
-// needs at most 64 entries and a two-level walk at most 128.
+// A binary radix tree over distinct 64-bit keys is at most 64 levels deep, so a walk needs at most 64
+// entries.
 constexpr int kMaxStack = 64;
-constexpr int kMaxStack2 = 128;
+// Words of work counters before the spill area.
+constexpr uint32_t kTraceHeaderWords = 256;
+
+// First of the next 64 rays of a wave of the one-ray-per-lane kernels: its own first, then from a counter
+// (zeroed when there are more rays than lanes; not read otherwise).
+__device__ __forceinline__ uint32_t next_rays(uint32_t *__restrict__ work, bool &first) {
+  const uint32_t lanes = gridDim.x * kTraceBlock;
+  uint32_t base = blockIdx.x * kTraceBlock + (threadIdx.x & ~63u);
+  if (!first) {
+    base = 0;
+    if ((threadIdx.x & 63) == 0) base = atomicAdd(work, 64u);
+    base = __builtin_amdgcn_readfirstlane(base);
+    base = base < ~0u - lanes ? base + lanes : ~0u;  // ~0: beyond any count
+  }
+  first = false;
+  return __builtin_amdgcn_readfirstlane(base);
+}
 
 // Closest hit so far. Hits are ordered by (t, inst, prim) with unsigned comparisons, so the
 // result does not depend on the order in which subtrees or instances are visited.
@@ -118,72 +133,14 @@ __device__ __forceinline__ void intersect_leaf(const RayPre &r, const TriRecord 
     intersect_record(r, rec, inst, tag, h);
 }
 
-// Depth-first walk of the subtree rooted at `start` (an inner node index, or ~leaf position) of a
-// tree with `nprims` leaves, using stack slots [sp0, MaxStack). leaf(position, spTop) is called
-// for every leaf whose box the ray meets; spTop is the first free stack slot. A child equal to
-// `skip` (a subtree already searched completely; kNoSkip for none) is not entered. Returns the
-// number of inner nodes fetched.
 constexpr int kNoSkip = INT_MIN;
 
-template <int MaxStack, class LeafFn>
-__device__ __forceinline__ uint32_t walk(const RayPre &r, const BVHNode *__restrict__ nodes, uint32_t nprims,
-                                         int start, const HitState &h, const LaneStack &st, int sp0, int skip,
-                                         LeafFn &&leaf) {
-  if (nprims == 0) return 0;  // an empty tree has no nodes
-  if (start < 0) {
-    leaf(~start, sp0);
-    return 0;
-  }
-  int node = start;
-  int sp = sp0;
-  uint32_t visits = 0;
-  // Each inner node is fetched at most once per walk; the step bound and the index check only
-  // guard against a malformed tree.
-  for (uint32_t step = 0; step < nprims; ++step) {
-    if ((uint32_t)node >= nprims - 1) break;
-    const BVHNode nd = nodes[node];
-    ++visits;
-    float tn0, tn1;
-    bool h0 = box_hit(r, nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y, h.t, tn0);
-    bool h1 = box_hit(r, nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w, h.t, tn1);
-    const int c0 = nd.d.x, c1 = nd.d.y;
-    h0 = h0 && c0 != skip;
-    h1 = h1 && c1 != skip;
-    if (h0 && c0 < 0) {
-      leaf(~c0, sp);
-      h0 = false;
-    }
-    if (h1 && c1 < 0) {
-      // The first leaf may have tightened h.t; the box test above used the older bound, which
-      // only costs a redundant leaf test.
-      leaf(~c1, sp);
-      h1 = false;
-    }
-    if (h0 && h1) {
-      const bool firstNear = tn0 <= tn1;
-      const int nearC = firstNear ? c0 : c1;
-      const int farC = firstNear ? c1 : c0;
-      if (sp < kLdsStack)
-        st.lds[sp][st.tid] = (uint32_t)farC;
-      else if (sp < MaxStack)
-        st.spill[sp - kLdsStack] = (uint32_t)farC;
-      ++sp;
-      node = nearC;
-    } else if (h0) {
-      node = c0;
-    } else if (h1) {
-      node = c1;
-    } else {
-      if (sp == sp0) break;
-      --sp;
-      if (sp >= MaxStack) break;  // unreachable within the depth bounds above
-      node = (int)stack_read(st, sp);
-    }
-  }
-  return visits;
-}
-
-// Depth-first walk like walk(), with leaf tests postponed and batched across the wave: a lane
+// Depth-first walk of the subtree rooted at `start` (an inner node index, or ~leaf position) of a
+// tree with `nprims` leaves, using stack slots [sp0, MaxStack). leaf(position, spTop) is called for
+// every leaf whose box the ray meets; spTop is the first free stack slot. A child equal to `skip` (a
+// subtree already searched completely; kNoSkip for none) is not entered.
+//
+// Leaf tests are postponed and batched across the wave: a lane
 // queues the leaf children it meets (up to kLeafQueue, in registers) and keeps walking; the wave
 // runs its leaf tests when at least half of its active lanes have leaves queued, or when a lane can
 // go no further (no node left, or no room for another node's two leaves). The triangle test is
@@ -193,9 +150,7 @@ __device__ __forceinline__ uint32_t walk(const RayPre &r, const BVHNode *__restr
 // result independent of the order of the tests. Returns the number of inner nodes fetched.
 constexpr int kLeafQueue = 4;
 
-// kPlain: no subtree is skipped and fetches are not counted (the walk returns 0), and the tree has
-// fewer than kSmallTreePrims primitives: the form of a plain trace, with fewer instructions per node.
-template <int MaxStack, class LeafFn, bool kPlain = false>
+template <int MaxStack, class LeafFn>
 __device__ __forceinline__ uint32_t walk_batched(const RayPre &r, const BVHNode *__restrict__ nodes, uint32_t nprims,
                                                  int start, const HitState &h, const LaneStack &st, int sp0, int skip,
                                                  LeafFn &&leaf) {
@@ -225,17 +180,14 @@ __device__ __forceinline__ uint32_t walk_batched(const RayPre &r, const BVHNode 
       if ((uint32_t)node >= nprims - 1) {
         node = kDone;  // only a malformed tree
       } else {
-        // node >= 0 here: no sign extension
-        const BVHNode nd = kPlain ? at32(nodes, (uint32_t)node) : nodes[(uint32_t)node];
-        if (!kPlain) ++visits;
+        const BVHNode nd = nodes[(uint32_t)node];  // node >= 0 here: no sign extension
+        ++visits;
         float tn0, tn1;
         bool h0 = box_hit(r, nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y, h.t, tn0);
         bool h1 = box_hit(r, nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w, h.t, tn1);
         const int c0 = nd.d.x, c1 = nd.d.y;
-        if (!kPlain) {
-          h0 = h0 && c0 != skip;
-          h1 = h1 && c1 != skip;
-        }
+        h0 = h0 && c0 != skip;
+        h1 = h1 && c1 != skip;
         if (h0 && c0 < 0) {
           enqueue(c0);
           h0 = false;
@@ -286,15 +238,431 @@ __device__ __forceinline__ uint32_t walk_batched(const RayPre &r, const BVHNode 
 
 // Primitive-accel walk: leaves are triangles (or, with kBoxes, box primitives) of instance `inst`;
 // `tag` is recorded with a hit.
-template <int MaxStack, bool kBoxes = false, bool kPlain = false>
+template <int MaxStack, bool kBoxes = false>
 __device__ __forceinline__ uint32_t traverse(const RayPre &r, const BVHNode *__restrict__ nodes,
                                              const TriRecord *__restrict__ tris, uint32_t nprims, int start,
                                              HitState &h, const LaneStack &st, int sp0, uint32_t inst, int tag,
                                              int skip = kNoSkip) {
   auto leafTest = [&](int leaf, int) __attribute__((always_inline)) {
-    intersect_leaf<kBoxes, kPlain>(r, tris, leaf, nprims, inst, tag, h);
+    intersect_leaf<kBoxes>(r, tris, leaf, nprims, inst, tag, h);
   };
-  return walk_batched<MaxStack, decltype(leafTest) &, kPlain>(r, nodes, nprims, start, h, st, sp0, skip, leafTest);
+  return walk_batched<MaxStack, decltype(leafTest) &>(r, nodes, nprims, start, h, st, sp0, skip, leafTest);
+}
+
+// A ray as the node test wants it. Per axis the distance to a plane p is p * i + b, b = -o * i: one FMA
+// instead of a subtraction and a multiplication. Its error beyond the relative ones (of i and of the
+// result, which the test's margin covers) is b's own rounding, at most 2^-24 |o * i|: the near plane's
+// b is lowered and the far plane's raised by twice that, which widens boxes by 2^-23 |o|, less than a
+// box's own coordinates near o are rounded. (One slack on the distances instead would let a ray with a
+// near-zero direction component, whose i is huge, enter every box.) Which plane is near follows from
+// the direction's sign, kept as lane masks. An axis whose products overflow is ignored.
+struct SlabRay {
+  float ix, iy, iz;  // reciprocal direction
+  float nx, ny, nz;  // b of the near planes
+  float fx, fy, fz;  // b of the far planes
+  float tmin;
+  bool px, py, pz;  // direction not negative: the near plane is the lower one
+};
+
+__device__ __forceinline__ void slab_axis(float o, float i, float &si, float &n, float &f, bool &p) {
+  const float b = -(o * i), e = fabsf(b) * 1.1920929e-07f;
+  const bool fine = fabsf(b) < 3.0e38f;
+  si = fine ? i : 0.0f;
+  n = fine ? b - e : -INFINITY;
+  f = fine ? b + e : INFINITY;
+  p = i >= 0.0f;
+}
+
+__device__ __forceinline__ SlabRay slab_ray(const RayPre &r) {
+  SlabRay s;
+  slab_axis(r.ox, r.ix, s.ix, s.nx, s.fx, s.px);
+  slab_axis(r.oy, r.iy, s.iy, s.ny, s.fy, s.py);
+  slab_axis(r.oz, r.iz, s.iz, s.nz, s.fz, s.pz);
+  s.tmin = r.tmin;
+  return s;
+}
+
+// Conservative test of a node's child box: accepted unless the later of its entry distance and tmin
+// exceeds the earlier of its exit distance and tbest by more than 2^-12 of the latter, far above the
+// rounding of the distances and of the primitive tests (the margin box_hit keeps). NaN distances are
+// ignored, so they accept. 18 vector instructions.
+__device__ __forceinline__ bool slab_hit(const SlabRay &r, float lox, float loy, float loz, float hix, float hiy,
+                                         float hiz, float tbest, float &tnear) {
+  const float nx = fmaf(r.px ? lox : hix, r.ix, r.nx), fx = fmaf(r.px ? hix : lox, r.ix, r.fx);
+  const float ny = fmaf(r.py ? loy : hiy, r.iy, r.ny), fy = fmaf(r.py ? hiy : loy, r.iy, r.fy);
+  const float nz = fmaf(r.pz ? loz : hiz, r.iz, r.nz), fz = fmaf(r.pz ? hiz : loz, r.iz, r.fz);
+  tnear = fmaxf(fmaxf(nx, ny), nz);
+  const float tf = fminf(fminf(fminf(fx, fy), fz), tbest);
+  return !(fmaxf(tnear, r.tmin) > fmaf(2.0f * kBoxSlack, fabsf(tf), tf));
+}
+
+
+// The plain trace: no proposal and no fetch counts. A wave keeps its 64 lanes busy. A lane whose ray has
+// ended gets the next one (with 64 fixed rays per wave, which walk until the longest one ends, 17 of 64
+// lanes are active on average), and once there is none left, a part of another lane's ray: the far subtree
+// at the bottom of its stack. The lanes fetch their nodes together.
+//
+// Node fetch: four lanes load one lane's node, 16 B each, into LDS (global_load_lds), for each of the
+// four lanes of the quad in turn; then every lane reads its node from LDS. Where each lane loads its
+// own node, every 16-byte load is one access of the vector cache, whose address and data paths were
+// busy 94 % of the time; the 64 contiguous bytes of a quad are one access for four lanes. Lane j loads
+// part j ^ k of the node of lane k of its quad, so that neighbouring lanes' reads of one part fall into
+// different banks. A lane without a node loads the root's.
+//
+// Rays: the waves of one XCD (workgroups are dealt to the eight XCDs in turn) take chunks of rays from
+// one contiguous share of them, so that its L2 holds what neighbouring rays meet (L2 misses 292 -> 222
+// million), then from the others' shares. A wave's first chunk is its own, the next ones are taken from a
+// counter per share, each on a line of its own: updates of one line by all CUs pass one at a time, about
+// 10 ns each (one counter for all cost 80 us for the first chunks alone). Chunks hold 64 rays (128 and
+// 256 measured no better), or, where that is less, an equal part of the rays for every wave, but two at
+// least (1 to 4 measured alike, 16 slower below 100,000 rays). A wave hands rays out when kRefill lanes
+// are free: 4 to 16 measured alike, 32 2 % slower.
+//
+// Split rays: a trace of few rays, and the end of one of many, otherwise waits for single lanes that walk
+// the longest rays (the longest meets 1,093 nodes, the average one 131). Hits are the minimum over (t,
+// inst, prim), so the parts of a ray may be walked in any order and by any lane; what order adds is the
+// bound, so the lanes of one ray share it. Every kSplitEvery steps with kSplitIdle idle lanes: 24 and 2
+// measured best of 8 to 64 and 1 to 16 (8 and 4: 8 % slower at 65,536 rays through 16,384 triangles).
+//
+// Times before and after, us, half primary and half bounce rays:
+//   through          512 rays     8,192       65,536      262,144     1,048,352    8,388,608
+//     16,384 tris   160 -> 40   185 -> 51   198 -> 69   226 -> 124    409 -> 277   2174 -> 1450
+//    262,144        270 -> 51   404 -> 70   443 -> 145  481 -> 326    941 -> 666   4844 -> 3400
+//  4,194,304        429 -> 62   584 -> 101  703 -> 226  811 -> 500   1610 -> 1134  7971 -> 5690
+// What bounds the largest now is the latency of the vector cache's misses (two thirds of the node fetches
+// miss L1, a third of those L2; the vector units are 58 % busy), the smallest the longest chain of nodes.
+constexpr int kRefill = 12;
+constexpr int kSplitIdle = 24;
+constexpr uint32_t kSplitEvery = 2;
+constexpr uint32_t kShares = 8;
+constexpr uint32_t kShareWords = 32;  // a counter's 128-byte line
+constexpr uint32_t kChunk = 64, kMinChunk = 2;
+static_assert(kShares * kShareWords <= kTraceHeaderWords, "the counters lie before the spill area");
+// 4 KB of nodes, 13 stack entries and the bounds per wave: 10 workgroups (20 waves) fit a CU. 11 entries
+// and 11 workgroups measured the same.
+constexpr int kStreamStack = 13;
+constexpr int kStreamBlocksPerCU = 10;
+static_assert((kMaxStack - kStreamStack) * kStreamBlocksPerCU <= (kMaxStack - kLdsStack) * kBlocksPerCU,
+              "the spill area is sized for the other kernels");
+
+struct StreamLds {
+  float4 node[kTraceBlock / 64][4 * 64];  // also scratch between two fetches
+  uint32_t stack[kStreamStack][kTraceBlock];
+  float best[kTraceBlock];  // split rays: closest hit distance so far, at the ray's owner
+};
+
+typedef __attribute__((address_space(3))) void LdsVoid;
+typedef __attribute__((address_space(1))) void GlobalVoid;
+
+__device__ __forceinline__ bool lane_of(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+__device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// The value of lane `src`; all lanes take part.
+template <class T>
+__device__ __forceinline__ T from_lane(const T &v, int src) {
+  static_assert(sizeof(T) % 4 == 0, "moved word by word");
+  int w[sizeof(T) / 4];
+  __builtin_memcpy(w, &v, sizeof(T));
+  for (int &x : w) x = __builtin_amdgcn_ds_bpermute(src * 4, x);
+  T out;
+  __builtin_memcpy(&out, w, sizeof(T));
+  return out;
+}
+
+// Keeps the LDS accesses of a wave's lanes, which the LDS executes in order, in program order.
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int K>
+__device__ __forceinline__ void fetch_quad_lane(const BVHNode *__restrict__ nodes, uint32_t at, uint32_t part,
+                                                char *stage) {
+  const uint32_t theirs = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)at, K * 0x55, 0xF, 0xF, true);
+  __builtin_amdgcn_global_load_lds((GlobalVoid *)((const char *)nodes + (theirs | (part ^ (K * 16u)))),
+                                   (LdsVoid *)(stage + K * 1024), 16, 0, 0);
+}
+
+// `at`: byte offset of the lane's node. All 64 lanes take part.
+__device__ __forceinline__ void fetch_nodes(const BVHNode *__restrict__ nodes, uint32_t at, char *stage) {
+  const uint32_t part = (threadIdx.x & 3u) * 16u;
+  fetch_quad_lane<0>(nodes, at, part, stage);
+  fetch_quad_lane<1>(nodes, at, part, stage);
+  fetch_quad_lane<2>(nodes, at, part, stage);
+  fetch_quad_lane<3>(nodes, at, part, stage);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Chunks of the rays, and of each share.
+struct Shares {
+  uint32_t chunk, chunks, seg;
+};
+__device__ __forceinline__ Shares shares_of(uint32_t count, uint32_t chunk) {
+  Shares s;
+  s.chunk = chunk;
+  s.chunks = (count - 1) / chunk + 1;
+  s.seg = (s.chunks - 1) / kShares + 1;
+  return s;
+}
+// Chunk c of share x, counted over all rays (beyond the last one if the share has no more).
+__device__ __forceinline__ uint32_t share_chunk(const Shares &s, uint32_t x, uint32_t c) {
+  return c < s.seg ? x * s.seg + c : 0xFFFFFFFFu;
+}
+// Chunks of share x that its own waves take first, one each.
+__device__ __forceinline__ uint32_t share_static(uint32_t x) {
+  return (gridDim.x + kShares - 1 - x) / kShares * (kTraceBlock / 64);
+}
+
+// The wave's next chunk: `left` rays from `next` on; false when all shares are used up. `share` counts
+// the shares that the wave found used up; their order differs between XCDs.
+__device__ __forceinline__ bool stream_chunk(uint32_t *__restrict__ work, uint32_t count, const Shares &s,
+                                             uint32_t &share, uint32_t &next, uint32_t &left) {
+  for (; share < kShares; ++share) {
+    const uint32_t x = (blockIdx.x ^ __builtin_bitreverse32(share << 29)) % kShares;
+    const uint32_t first = share_static(x);
+    uint32_t c = share_chunk(s, x, first);
+    if (c < s.chunks) {
+      uint32_t base = 0;
+      if ((threadIdx.x & 63) == 0) base = atomicAdd(work + kShareWords * x, 1u);
+      c = share_chunk(s, x, first + __builtin_amdgcn_readfirstlane(base));
+      if (c < s.chunks) {
+        next = c * s.chunk;
+        left = min(s.chunk, count - next);
+        return true;
+      }
+    }
+  }
+  return false;
+}
+
+// Split rays: `own` is the lane that holds the ray's hit, itself for a lane without a part of another's.
+// Takes the hits of the lanes that have ended their parts to the owners (the closest one by the rule of
+// hit_closer: first the distance, then instance and primitive) and tells at stage + kSplitActive, a word
+// per lane, whether a lane that still walks belongs to the owner. All 64 lanes take part.
+constexpr int kSplitActive = 1792;
+
+__device__ __forceinline__ void settle_parts(char *stage, int lane, int own, bool busy, HitState &h) {
+  uint32_t *sT = (uint32_t *)stage;
+  unsigned long long *sKey = (unsigned long long *)(stage + 256);
+  float *sHitT = (float *)(stage + 768), *sU = (float *)(stage + 1024), *sV = (float *)(stage + 1280);
+  int *sLeaf = (int *)(stage + 1536);
+  uint32_t *sActive = (uint32_t *)(stage + kSplitActive);
+  const bool hit = h.prim >= 0, owner = own == lane;
+  const uint32_t t = hit ? ford(h.t + 0.0f) : ~0u;  // + 0: distances -0 and +0 are equal
+  const unsigned long long key = hit ? ((unsigned long long)h.inst << 32 | (uint32_t)h.prim) : ~0ull;
+  lds_order();
+  sT[lane] = owner ? t : ~0u;
+  sKey[lane] = owner ? key : ~0ull;
+  sActive[lane] = 0;
+  lds_order();
+  const bool found = !busy && !owner && hit;
+  if (found) atomicMin(&sT[own], t);
+  if (busy) sActive[own] = 1;
+  lds_order();
+  const bool closest = found && sT[own] == t;
+  if (owner && sT[lane] != t) sKey[lane] = ~0ull;
+  lds_order();
+  if (closest) atomicMin(&sKey[own], key);
+  lds_order();
+  if (closest && sKey[own] == key) {
+    sHitT[own] = h.t;
+    sU[own] = h.u;
+    sV[own] = h.v;
+    sLeaf[own] = h.leaf;
+  }
+  lds_order();
+  if (owner && (sT[lane] != t || sKey[lane] != key)) {
+    h.t = sHitT[lane];
+    h.u = sU[lane];
+    h.v = sV[lane];
+    h.leaf = sLeaf[lane];
+    h.prim = (int)(uint32_t)sKey[lane];
+    h.inst = (uint32_t)(sKey[lane] >> 32);
+  }
+}
+
+// Traces rays [0, count), `chunk` at a time: begin(i) sets up ray i in the caller's `ray`, `slab` and `h`,
+// leaf(position) tests a leaf, end(i) stores ray i's hit. `work`: kShares counters, zeroed (read only if
+// there are more chunks than waves), kShareWords apart. `spill`: this lane's kMaxStack - kStreamStack
+// words. The tree has fewer than kSmallTreePrims primitives.
+template <class Begin, class Leaf, class End>
+__device__ __forceinline__ void trace_stream(const BVHNode *__restrict__ nodes, uint32_t nprims, uint32_t count,
+                                             uint32_t chunk, uint32_t *__restrict__ work, RayPre &ray, SlabRay &slab,
+                                             HitState &h, StreamLds &lds, uint32_t *__restrict__ spill, Begin &&begin,
+                                             Leaf &&leaf, End &&end) {
+  constexpr uint32_t kDone = 0x80000000u, kNoRay = 0xFFFFFFFFu;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const uint32_t waveInBlock = __builtin_amdgcn_readfirstlane(tid >> 6);
+  char *stage = (char *)lds.node[waveInBlock];
+  float *best = lds.best + waveInBlock * 64;
+  const uint32_t quad = tid & 3u;
+  const char *mine = stage + quad * 1024u + (tid & 60u) * 16u;
+  // Queued leaves as child codes, as in walk_batched.
+  int q0 = -1, q1 = -1, q2 = -1, q3 = -1, nq = 0;
+  auto enqueue = [&](int code) __attribute__((always_inline)) {
+    q3 = q2;
+    q2 = q1;
+    q1 = q0;
+    q0 = code;
+    ++nq;
+  };
+  const uint32_t inner = nprims > 1 ? nprims - 1 : 0u;  // a node at or above it: none (or a malformed tree)
+  // In every iteration a lane with a ray fetches a node (each at most once) or tests its queued leaves.
+  const uint32_t limit = 4u * nprims + 8u;
+  uint32_t ri = kNoRay, began = 0, node = kDone;
+  int own = lane;
+  int sp = 0, bot = 0;  // the stack's entries are [bot, sp)
+  // Wave-uniform: the chunk's remaining rays, and which lanes have a node to visit and queued leaves.
+  const Shares shares = shares_of(count, chunk);
+  uint32_t share = 0, next = 0, left = 0;
+  const uint32_t c = share_chunk(shares, blockIdx.x % kShares, blockIdx.x / kShares * (kTraceBlock / 64) + waveInBlock);
+  if (c < shares.chunks) {
+    next = c * chunk;
+    left = min(chunk, count - next);
+  }
+  bool more = true;
+  uint64_t walk = 0, wait = 0;
+  for (uint32_t it = 0;; ++it) {
+    const uint64_t idle = ~(walk | wait);
+    if (__builtin_expect(more && __popcll(idle) >= kRefill, 0)) {
+      const bool free = lane_of(idle);
+      if (free && ri != kNoRay) {
+        end(ri);
+        ri = kNoRay;
+      }
+      if (left == 0) more = stream_chunk(work, count, shares, share, next, left);
+      if (!more) {
+        best[lane] = h.t;
+        continue;
+      }
+      const uint32_t rank = lane_rank(idle);
+      if (free && rank < left) {
+        ri = next + rank;
+        begin(ri);
+        began = it;
+        sp = bot = 0;
+        if (inner > 0)
+          node = 0;
+        else if (nprims == 1)
+          enqueue(~0);
+      }
+      const uint32_t took = min((uint32_t)__popcll(idle), left);
+      next += took;
+      left -= took;
+      walk = __ballot(node < inner);
+      wait = __ballot(nq > 0);
+    }
+    if (!more && __builtin_expect(idle == ~0ull || (__popcll(idle) >= kSplitIdle && it % kSplitEvery == 0), 0)) {
+      const bool busy = !lane_of(idle);
+      settle_parts(stage, lane, own, busy, h);
+      if (!busy) {
+        if (own == lane && ri != kNoRay && ((const uint32_t *)(stage + kSplitActive))[lane] == 0) {
+          end(ri);
+          ri = kNoRay;
+        } else if (own != lane) {
+          ri = kNoRay;
+          own = lane;
+        }
+      }
+      if (idle == ~0ull) break;
+      // The k-th lane that gives takes the bottom of its stack to the k-th free lane.
+      const bool free = !busy && ri == kNoRay, gives = busy && sp > bot && bot < kStreamStack;
+      const uint64_t frees = __ballot(free), givers = __ballot(gives);
+      if (frees && givers) {
+        const uint32_t toRank = lane_rank(frees), fromRank = lane_rank(givers);
+        uint32_t *from = (uint32_t *)stage, *entry = from + 64;
+        lds_order();
+        if (gives && fromRank < (uint32_t)__popcll(frees)) {
+          from[fromRank] = lane;
+          entry[fromRank] = lds.stack[bot][tid];
+          ++bot;
+        }
+        lds_order();
+        const bool takes = free && toRank < (uint32_t)__popcll(givers);
+        const int src = takes ? (int)from[toRank] : lane;
+        const RayPre theirs = from_lane(ray, src);
+        const uint32_t theirRi = from_lane(ri, src);
+        const int theirOwn = from_lane(own, src);
+        if (takes) {
+          ray = theirs;
+          slab = slab_ray(ray);
+          ri = theirRi;
+          own = theirOwn;
+          hit_init(h, best[own]);
+          node = entry[toRank];
+          began = it;
+          sp = bot = 0;
+        }
+        walk = __ballot(node < inner);
+        lds_order();
+      }
+    }
+    if ((it & 4095u) == 4095u) {
+      if (it - began > limit) {  // only a malformed tree
+        node = kDone;
+        nq = 0;
+      }
+      walk = __ballot(node < inner);
+      wait = __ballot(nq > 0);
+    }
+    if (walk) fetch_nodes(nodes, lane_of(walk) ? node * (uint32_t)sizeof(BVHNode) : 0u, stage);
+    if (lane_of(walk)) {
+      const float4 a = *(const float4 *)(mine + (0u ^ quad) * 16u), b = *(const float4 *)(mine + (1u ^ quad) * 16u);
+      const float4 d = *(const float4 *)(mine + (2u ^ quad) * 16u);
+      const int2 child = *(const int2 *)(mine + (3u ^ quad) * 16u);
+      float tn0, tn1, bound = h.t;
+      if (!more) bound = fminf(bound, best[own]);
+      // Lane masks rather than flags: they stay in scalar registers.
+      const uint64_t h0 = __ballot(slab_hit(slab, a.x, a.y, a.z, a.w, b.x, b.y, bound, tn0));
+      const uint64_t h1 = __ballot(slab_hit(slab, b.z, b.w, d.x, d.y, d.z, d.w, bound, tn1));
+      const uint64_t n0 = __ballot(child.x >= 0), n1 = __ballot(child.y >= 0), near0 = __ballot(tn0 <= tn1);
+      const uint64_t i0 = h0 & n0, i1 = h1 & n1, l0 = h0 & ~n0, l1 = h1 & ~n1;
+      if (lane_of(l0 | l1)) {
+        enqueue(lane_of(l0) ? child.x : child.y);
+        if (lane_of(l0 & l1)) enqueue(child.y);
+      }
+      const bool first0 = lane_of(i0 & (~i1 | near0));
+      node = (uint32_t)(first0 ? child.x : child.y);
+      if (lane_of(i0 & i1)) {
+        const uint32_t other = (uint32_t)(first0 ? child.y : child.x);
+        if (sp < kStreamStack)
+          lds.stack[sp][tid] = other;
+        else if (sp < kMaxStack)
+          spill[sp - kStreamStack] = other;
+        ++sp;
+      }
+      if (lane_of(~(i0 | i1))) {
+        node = kDone;
+        if (sp != bot) {
+          --sp;
+          if (sp < kStreamStack)
+            node = lds.stack[sp][tid];
+          else if (sp < kMaxStack)  // an ordinary load: see stack_read
+            node = __hip_atomic_load(&spill[sp - kStreamStack], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        }
+      }
+    }
+    walk = __ballot(node < inner);
+    wait = __ballot(nq > 0);
+    // A lane that walks no further, or has no room for another node's two leaves (so that no queue is ever
+    // full at the top of the loop), needs its leaves tested.
+    if ((wait & (~walk | __ballot(nq > kLeafQueue - 2))) || 2 * __popcll(wait) >= __popcll(walk | wait)) {
+      while (nq > 0) {
+        const int code = q0;
+        q0 = q1;
+        q1 = q2;
+        q2 = q3;
+        --nq;
+        leaf(~code);
+      }
+      if (!more && lane_of(wait))
+        __hip_atomic_fetch_min(&best[own], h.t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      wait = 0;
+    }
+  }
 }
 
 }  // namespace gprt

@@ -303,3 +303,35 @@ def test_plain_and_general_trace_forms_agree(ctx):
     assert min(hits) > 0.02  # the comparison covers hits, not only misses
     for a in [tlas, box, tri] + blas:
         a.destroy()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 65, 6000])
+@pytest.mark.parametrize("rays", [1, 2, 63, 4097, 20481, 400001])
+def test_streamed_trace_equals_general_form(ctx, n, rays):
+    """A plain trace hands out rays in chunks and splits them between lanes; asking for fetch counts
+    traces one ray per lane. Bit-identical hits: fewer rays than waves, ragged chunks, and more rays
+    than a launch takes at once; every triangle twice, so that parts of a split ray end in ties; on a
+    triangle accel and on an instance accel that holds it twice, in place and moved."""
+    verts, idx = scenes.uniform_scene((n + 1) // 2, seed=40 + n)
+    idx = np.ascontiguousarray(np.concatenate([idx, idx])[:n])
+    acc = _build(ctx, verts, idx)
+    moved = np.eye(3, 4, dtype=np.float32)
+    moved[:, 3] = np.float32(0.05)
+    same = np.eye(3, 4, dtype=np.float32)
+    tlas = api.InstanceAccel(ctx, api.instance_records([acc, acc, acc], transforms=[same, moved, same]))
+    tlas.build()
+    r = scenes.random_rays(rays, seed=n + rays)
+    r["tmax"][::5] = np.float32(0.3)
+    rb, vb = ctx.device_buffer(r), ctx.device_buffer(nbytes=4 * rays)
+    h1, h2 = ctx.device_buffer(nbytes=16 * rays), ctx.device_buffer(nbytes=16 * rays)
+    i1, i2 = ctx.device_buffer(nbytes=4 * rays), ctx.device_buffer(nbytes=4 * rays)
+    for a in (acc, tlas):
+        api.trace_detail(ctx, a, rb, h1, rays, i1)
+        api.trace_detail(ctx, a, rb, h2, rays, i2, visits_buf=vb)
+        assert api.last_error() is None, api.last_error()
+        _assert_hits_equal(h1.read(api.HIT_DTYPE), h2.read(api.HIT_DTYPE))
+        np.testing.assert_array_equal(i1.read(np.int32), i2.read(np.int32))
+    for b in (rb, vb, h1, h2, i1, i2):
+        b.destroy()
+    tlas.destroy()
+    acc.destroy()
