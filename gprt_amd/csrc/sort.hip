@@ -16,6 +16,8 @@
 //    sort can be captured in a hipGraph.
 // Up to 16,384 keys, where those launches would be all the time there is, k_rank places every key by
 // comparing it with all others and k_copy_pairs puts the result back: two launches.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "internal.hpp"
 
@@ -206,11 +208,9 @@ __global__ void __launch_bounds__(THREADS)
     k[j] = idx < n ? src[idx] : ~(KT)0;
     d[j] = digit_of(k[j], shift, dmask);
   }
-  // 32-bit payloads of 32-bit keys are loaded with the keys, so their loads overlap the ranking and
-  // the look-back (the registers fit without lowering occupancy); wider ones after the key write.
-  constexpr bool kEarlyVals = VB == 32 && sizeof(KT) == 4;
-  VT ve[kEarlyVals ? ITEMS : 1];
-  if constexpr (kEarlyVals) {
+  // The payloads are loaded with the keys, so their loads overlap the ranking and the look-back.
+  VT ve[VB ? ITEMS : 1];
+  if constexpr (VB != 0) {
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
       const size_t idx = waveBase + (size_t)j * 64 + l;
@@ -336,18 +336,11 @@ __global__ void __launch_bounds__(THREADS)
     if ((uint32_t)(j * THREADS + tid) < valid && gaddr[j] < n) dst[gaddr[j]] = sk[j];
   }
 
-  if (VB) {
+  if constexpr (VB != 0) {
     __syncthreads();
     VT *s_vals = (VT *)s_buf;
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      if constexpr (kEarlyVals) {
-        s_vals[pos[j]] = ve[j];
-      } else {
-        const size_t idx = waveBase + (size_t)j * 64 + l;
-        s_vals[pos[j]] = idx < n ? vsrc[idx] : (VT)0;
-      }
-    }
+    for (int j = 0; j < ITEMS; ++j) s_vals[pos[j]] = ve[j];
     __syncthreads();
     VT sv[ITEMS];
 #pragma unroll
@@ -460,18 +453,28 @@ void run_rank(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAlt
 
 inline int passes_for(int loBit, int hiBit, int bits) { return (hiBit - loBit + bits - 1) / bits; }
 
-// Keys per tile of one sort: 2,048 when asked for; 4,096 for 64-bit keys or payloads (their
-// larger tiles do not fit the LDS); automatically 16,384 (1,024 threads x 16) for at least 2^22
-// narrow keys and 8,192 below (fewer, larger tiles cost fewer look-back steps once every CU has
-// tiles to rank); otherwise the configured size.
-constexpr size_t kAutoLargeTileKeys = (size_t)1 << 22;
+// Keys per tile of one sort. Automatically 2,048 (256 threads x 8) up to 2^18 keys, where a pass is as long
+// as one tile takes; 4,096 (256 x 16) for 64-bit keys or payloads and 8,192 (512 x 16) for narrow ones; and
+// 16,384 (1,024 x 16) from 1.5 million 64-bit keys, 2.6 million 64-bit payloads or 4 million narrow keys on,
+// where longer digit runs and fewer look-back steps count more. Us, with the smaller against the larger tile: 60,000 64-bit pairs 105 against 147, 260,000 134
+// against 173, 400,000 151 against 145; 60,000 32-bit pairs 66 against 79, 400,000 89 against 87; 1 million
+// 64-bit pairs 193 against 273, 4 million 439 against 362, 16 million 1508 against 1466, keys alone 176
+// against 200, 360 against 261, 944 against 749; 2 million pairs 270 against 301, keys 241 against 220. Asked for: 2,048, 4,096, and with narrow keys 8,192 and
+// 16,384 are taken as they are, with wide ones as 4,096.
+// (Payloads used to be loaded after the ranking where a key or payload has 64 bits: 16 million 64-bit pairs
+// 1775, now 1504 in tiles of the same size.)
+constexpr size_t kAutoSmallTileKeys = (size_t)1 << 18;
+constexpr size_t large_tile_keys(int keyBits, int valBits) {
+  return valBits == 64 ? (size_t)5 << 19 : keyBits == 64 ? (size_t)3 << 19 : (size_t)1 << 22;
+}
 
 int tile_keys_effective(const SortConfig &cfg, size_t n, int keyBits, int valBits) {
   const bool wide = keyBits == 64 || valBits == 64;
-  if (cfg.tileKeys == 2048) return 2048;
-  if (wide) return 4096;  // 256 threads x 16 keys of 64 bits fit the LDS; 4,096 to 16,384 asked: 4,096
-  if (cfg.tileKeys == 0) return n >= kAutoLargeTileKeys ? 16384 : 8192;
-  return cfg.tileKeys;
+  if (cfg.tileKeys == 0) {
+    if (n <= kAutoSmallTileKeys) return 2048;
+    return n >= large_tile_keys(keyBits, valBits) ? 16384 : wide ? 4096 : 8192;
+  }
+  return wide ? std::min(cfg.tileKeys, 4096) : cfg.tileKeys;
 }
 
 template <typename KT, int VB, int BITS, int THREADS, int ITEMS>
@@ -506,22 +509,16 @@ void run_typed(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAl
 template <typename KT, int VB, int BITS>
 bool run_bits(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAlt, void *valsAlt, size_t n, int loBit,
               int hiBit, void *scratch, const SortConfig &cfg) {
-  constexpr bool wide = sizeof(KT) == 8 || VB == 64;
   switch (tile_keys_effective(cfg, n, (int)sizeof(KT) * 8, VB)) {
     case 2048: run_typed<KT, VB, BITS, 256, 8>(ctx, s, keys, vals, keysAlt, valsAlt, n, loBit, hiBit, scratch); return true;
     case 4096: run_typed<KT, VB, BITS, 256, 16>(ctx, s, keys, vals, keysAlt, valsAlt, n, loBit, hiBit, scratch); return true;
     case 8192:
-      if constexpr (!wide) {
+      if constexpr (sizeof(KT) == 4 && VB <= 32) {
         run_typed<KT, VB, BITS, 512, 16>(ctx, s, keys, vals, keysAlt, valsAlt, n, loBit, hiBit, scratch);
         return true;
       }
       break;
-    case 16384:
-      if constexpr (!wide) {
-        run_typed<KT, VB, BITS, 1024, 16>(ctx, s, keys, vals, keysAlt, valsAlt, n, loBit, hiBit, scratch);
-        return true;
-      }
-      break;
+    case 16384: run_typed<KT, VB, BITS, 1024, 16>(ctx, s, keys, vals, keysAlt, valsAlt, n, loBit, hiBit, scratch); return true;
   }
   fail("sort: tileKeys %d is not one of 0, 2048, 4096, 8192, 16384", cfg.tileKeys);
   return false;
@@ -547,8 +544,12 @@ bool run_kv(Context *ctx, hipStream_t s, void *keys, void *vals, void *keysAlt, 
 size_t sort_scratch_bytes(size_t n, int keyBits, int valBits, int loBit, int hiBit, const SortConfig &cfg) {
   const int R = 1 << cfg.digitBits;
   const int passes = passes_for(loBit, hiBit, cfg.digitBits);
-  const size_t tile = (size_t)tile_keys_effective(cfg, n, keyBits, valBits);
-  const size_t tiles = (n + tile - 1) / tile;
+  // Not less than for fewer keys, whose tiles may be smaller: scratch for n keys does for all up to n.
+  size_t tiles = 0;
+  for (size_t m : {n, std::min(n, kAutoSmallTileKeys), std::min(n, large_tile_keys(keyBits, valBits) - 1)}) {
+    const size_t tile = (size_t)tile_keys_effective(cfg, m, keyBits, valBits);
+    tiles = std::max(tiles, (m + tile - 1) / tile);
+  }
   return ((size_t)passes * R + 32 + (size_t)passes * tiles * R) * 4;
 }
 
