@@ -241,6 +241,24 @@ def test_sort_by_ranks(ctx, n, kdt, vdt):
         np.testing.assert_array_equal(v, vals[order])
 
 
+# Either side of the sizes at which the tile changes (2,048, then 4,096 or 8,192, then 16,384 keys): ragged
+# last tiles, duplicates, and the largest key, which also pads the last tile.
+@pytest.mark.parametrize("kdt,vdt,n", [(np.uint32, np.uint32, (1 << 18) + d) for d in (0, 1)] +
+                         [(np.uint64, None, (3 << 19) + d) for d in (-1, 0)] +
+                         [(np.uint64, np.uint32, (3 << 19) + 16385), (np.uint64, np.uint64, (5 << 19) - 1),
+                          (np.uint64, np.uint64, (5 << 19) + 1), (np.uint32, np.uint64, (5 << 19) + 3)])
+def test_sort_around_tile_sizes(ctx, kdt, vdt, n):
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, n // 2, n).astype(kdt) * kdt(np.iinfo(kdt).max // (n // 2))
+    keys[::5] = np.iinfo(kdt).max
+    vals = None if vdt is None else np.arange(n, dtype=vdt)
+    k, v = _sort_kv(ctx, keys, vals)
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(k, keys[order])
+    if vals is not None:
+        np.testing.assert_array_equal(v, vals[order])
+
+
 def test_sort_constant_and_single_digit_keys(ctx, orc):
     n = 50_000
     # every digit constant: all passes skipped, data untouched
