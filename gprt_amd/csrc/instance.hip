@@ -801,7 +801,7 @@ bool tlas_trace(Context *ctx, hipStream_t s, Accel *a, const void *rays, void *h
   const bool checked = t->builtEpoch != ctx->blasEpoch;
   const char *name = proposal ? "trace_closest_proposal_instances" : "trace_closest_instances";
   const bool plain = !proposal && !visits && t->leaves < kSmallTreePrims;
-  const TraceGrid g = trace_grid(ctx, count, plain, blocksPerCU);
+  const TraceGrid g = trace_grid(ctx, t->leaves, count, plain, blocksPerCU);
   if (g.counters) fill_u32(ctx, s, work, 0u, g.counters);
   if (plain) {
     auto go = [&](auto kernel) {

@@ -304,7 +304,7 @@ struct TraceGrid {
   uint32_t counters;  // words of the scratch's head to zero before the launch
   uint32_t chunk;     // plain: rays a wave takes at a time
 };
-TraceGrid trace_grid(const Context *ctx, uint32_t count, bool plain, unsigned blocksPerCU);
+TraceGrid trace_grid(const Context *ctx, uint32_t n, uint32_t count, bool plain, unsigned blocksPerCU);
 // Work counters (first kTraceHeaderWords words) + per-lane stack spill of `spillWordsPerLane` words.
 uint32_t *ensure_trace_scratch(Context *ctx, hipStream_t s, int spillWordsPerLane);
 

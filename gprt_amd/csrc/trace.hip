@@ -124,16 +124,20 @@ uint32_t *ensure_trace_scratch(Context *ctx, hipStream_t s, int spillWordsPerLan
   return (uint32_t *)ctx->traceScratch;
 }
 
-// How `count` rays are traced. Plain: trace_stream by a full launch, in chunks of equal size for every
-// wave up to kChunk, and without counters where that leaves no chunk over. General: one ray per lane, in as
+// How `count` rays are traced through a tree of n leaves. Plain: trace_stream by a full launch, in one chunk
+// of equal size for every wave where that holds at most kChunk rays (and then without counters), else in
+// chunks of half of kChunk for large trees, whose rays differ most (us for 0.52 / 1.05 / 8.4 million rays
+// in chunks of 64 and 32: 4.2 million triangles 798 / 1141 / 5661 and 690 / 1068 / 5583, 262,144 461 / 649 /
+// 3360 and 403 / 625 / 3341; 16,384 196 / 268 / 1455 and 196 / 285 / 1495). General: one ray per lane, in as
 // many workgroups as that needs (a full launch of waves that each ask a counter cost 80 us), persistent
 // beyond a full launch.
-TraceGrid trace_grid(const Context *ctx, uint32_t count, bool plain, unsigned blocksPerCU) {
+TraceGrid trace_grid(const Context *ctx, uint32_t n, uint32_t count, bool plain, unsigned blocksPerCU) {
   const unsigned perCU = blocksPerCU ? blocksPerCU : UINT_MAX;
   if (plain) {
     const unsigned blocks = (unsigned)ctx->cuCount * std::min<unsigned>(perCU, kStreamBlocksPerCU);
     const uint32_t waves = blocks * (kTraceBlock / 64);
-    const uint32_t chunk = std::min(kChunk, std::max(kMinChunk, (count - 1) / waves + 1));
+    const uint32_t even = std::max(kMinChunk, (count - 1) / waves + 1);
+    const uint32_t chunk = even <= kChunk ? even : n < 1u << 16 ? kChunk : kChunk / 2;
     // Of each share's waves and chunks (trace_stream's numbers).
     const uint32_t least = blocks / kShares * (kTraceBlock / 64), seg = (count - 1) / chunk / kShares + 1;
     return TraceGrid{blocks, seg <= least ? 0u : kShares * kShareWords, chunk};
@@ -150,7 +154,7 @@ bool trace_closest_ex(Context *ctx, hipStream_t s, Accel *a, const void *rays, v
   uint32_t *work = ensure_trace_scratch(ctx, s, kMaxStack - kLdsStack);
   if (!work) return false;
   const bool plain = !proposal && !visits && a->n < kSmallTreePrims;
-  const TraceGrid g = trace_grid(ctx, count, plain, blocksPerCU);
+  const TraceGrid g = trace_grid(ctx, a->n, count, plain, blocksPerCU);
   if (g.counters) fill_u32(ctx, s, work, 0u, g.counters);
   if (plain) {
     auto go = [&](auto kernel) {

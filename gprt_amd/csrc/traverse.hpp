@@ -313,9 +313,9 @@ __device__ __forceinline__ bool slab_hit(const SlabRay &r, float lox, float loy,
 // one contiguous share of them, so that its L2 holds what neighbouring rays meet (L2 misses 292 -> 222
 // million), then from the others' shares. A wave's first chunk is its own, the next ones are taken from a
 // counter per share, each on a line of its own: updates of one line by all CUs pass one at a time, about
-// 10 ns each (one counter for all cost 80 us for the first chunks alone). Chunks hold 64 rays (128 and
-// 256 measured no better), or, where that is less, an equal part of the rays for every wave, but two at
-// least (1 to 4 measured alike, 16 slower below 100,000 rays). A wave hands rays out when kRefill lanes
+// 10 ns each (one counter for all cost 80 us for the first chunks alone). Chunks hold 64 rays or
+// 32 (128 and 256 measured no better), or, where that is less, an equal part of the rays for every wave, but
+// two at least (1 to 4 measured alike, 16 slower below 100,000 rays). A wave hands rays out when kRefill lanes
 // are free: 4 to 16 measured alike, 32 2 % slower.
 //
 // Split rays: a trace of few rays, and the end of one of many, otherwise waits for single lanes that walk
