@@ -613,6 +613,8 @@ __device__ __forceinline__ void trace_stream(const BVHNode *__restrict__ nodes, 
       const float4 a = *(const float4 *)(mine + (0u ^ quad) * 16u), b = *(const float4 *)(mine + (1u ^ quad) * 16u);
       const float4 d = *(const float4 *)(mine + (2u ^ quad) * 16u);
       const int2 child = *(const int2 *)(mine + (3u ^ quad) * 16u);
+      // The stack's top, should both children fail: read ahead, so that no step waits for it.
+      uint32_t top = lds.stack[min((uint32_t)sp - 1u, kStreamStack - 1u)][tid];
       float tn0, tn1, bound = h.t;
       if (!more) bound = fminf(bound, best[own]);
       // Lane masks rather than flags: they stay in scalar registers.
@@ -624,26 +626,23 @@ __device__ __forceinline__ void trace_stream(const BVHNode *__restrict__ nodes, 
         enqueue(lane_of(l0) ? child.x : child.y);
         if (lane_of(l0 & l1)) enqueue(child.y);
       }
-      const bool first0 = lane_of(i0 & (~i1 | near0));
-      node = (uint32_t)(first0 ? child.x : child.y);
-      if (lane_of(i0 & i1)) {
-        const uint32_t other = (uint32_t)(first0 ? child.y : child.x);
-        if (sp < kStreamStack)
-          lds.stack[sp][tid] = other;
-        else if (sp < kMaxStack)
-          spill[sp - kStreamStack] = other;
-        ++sp;
+      const uint64_t first0 = i0 & (~i1 | near0), push = i0 & i1;
+      const uint64_t pop = walk & ~(i0 | i1) & __ballot(sp != bot);
+      const uint64_t below = __ballot(sp < kStreamStack), above = __ballot(sp > kStreamStack);
+      if (lane_of(push & below)) lds.stack[sp][tid] = (uint32_t)(lane_of(first0) ? child.y : child.x);
+      if (__builtin_expect(push & ~below, 0)) {
+        if (lane_of(push & ~below) && sp < kMaxStack)
+          spill[sp - kStreamStack] = (uint32_t)(lane_of(first0) ? child.y : child.x);
       }
-      if (lane_of(~(i0 | i1))) {
-        node = kDone;
-        if (sp != bot) {
-          --sp;
-          if (sp < kStreamStack)
-            node = lds.stack[sp][tid];
-          else if (sp < kMaxStack)  // an ordinary load: see stack_read
-            node = __hip_atomic_load(&spill[sp - kStreamStack], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        }
+      if (__builtin_expect(pop & above, 0)) {
+        if (lane_of(pop & above))  // an ordinary load: see stack_read
+          top = sp <= kMaxStack ? __hip_atomic_load(&spill[sp - 1 - kStreamStack], __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_WAVEFRONT)
+                                : kDone;
       }
+      node = (uint32_t)(lane_of(first0) ? child.x : child.y);
+      node = lane_of(i0 | i1) ? node : lane_of(pop) ? top : kDone;
+      sp += (lane_of(push) ? 1 : 0) - (lane_of(pop) ? 1 : 0);
     }
     walk = __ballot(node < inner);
     wait = __ballot(nq > 0);
