@@ -155,13 +155,47 @@ struct ValType<64> {
   using T = uint64_t;
 };
 
+// Writes element `at` of fewer than 2^30: 32-bit offsets of 32-bit elements need one register less.
+template <typename T>
+__device__ __forceinline__ void put_at(T *base, uint32_t at, T v) {
+  if constexpr (sizeof(T) == 4)
+    *(T *)((char *)base + at * 4u) = v;
+  else
+    base[at] = v;
+}
+
+// A lane's ITEMS elements of a wave's consecutive ones, of which the first `here` exist (all if `whole`).
+template <int ITEMS, typename T>
+__device__ __forceinline__ void load_items(const T *__restrict__ p, bool whole, uint32_t here, T none, T (&out)[ITEMS]) {
+  const uint32_t l = threadIdx.x & 63u;
+  if (whole) {
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) out[j] = p[j * 64u + l];
+  } else {
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) out[j] = j * 64u + l < here ? p[j * 64u + l] : none;
+  }
+}
+
+// A pass alternates between memory (its loads, the look-back, its writes) and ranking, which keeps the
+// vector units busy for a third of the time (14,000 of 45,000 cycles a tile of 16,384); two workgroups of
+// 1,024 threads a CU overlap the two. That takes 64 registers per thread and 80 KB of LDS: 16-bit wave
+// counts and positions, digits computed again rather than kept, payloads loaded once the keys are in LDS,
+// few writes at a time, and a compiler that is kept from mixing the ranking of several keys and from
+// holding both halves of a pair of positions. Wider keys or payloads fill the LDS with one workgroup. A copy
+// of the input and the sort, us: 67 million 32-bit pairs 1597 -> 1472, keys 1195 -> 970, 16 million pairs
+// 443 -> 378; 16 million 64-bit pairs 1477 -> 1267 (fewer registers).
+template <typename KT, int VB, int THREADS>
+constexpr bool kTwoPerCU = THREADS == 1024 && sizeof(KT) == 4 && VB <= 32;
+
 template <typename KT, int VB, int BITS, int THREADS, int ITEMS>
-__global__ void __launch_bounds__(THREADS)
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(kTwoPerCU<KT, VB, THREADS> ? 8 : 1)))
     k_onesweep(KT *__restrict__ keys0, KT *__restrict__ keys1, void *__restrict__ vals0, void *__restrict__ vals1,
                uint32_t n, int pass, int shift, int hiBit, void *__restrict__ stateBase, int passes,
                uint32_t numTiles) {
   using VT = typename ValType<VB>::T;
   constexpr int R = 1 << BITS;
+  constexpr int NB = VB && kTwoPerCU<KT, VB, THREADS> ? 2 : 8;  // keys per thread written at a time: more need more registers
   constexpr int W = THREADS / 64;
   constexpr int TILE = THREADS * ITEMS;
   constexpr int DPT = (R + THREADS - 1) / THREADS;  // digits per thread
@@ -170,7 +204,7 @@ __global__ void __launch_bounds__(THREADS)
   constexpr size_t BUFBYTES = KBYTES > VBYTES ? KBYTES : VBYTES;
 
   __shared__ __attribute__((aligned(16))) unsigned char s_buf[BUFBYTES];
-  __shared__ uint32_t s_whist[W][R];
+  __shared__ uint16_t s_whist[W][R];
   __shared__ uint32_t s_tdigit[R];
   __shared__ uint32_t s_gbase[R];
   __shared__ uint32_t s_wtot[W];
@@ -186,47 +220,46 @@ __global__ void __launch_bounds__(THREADS)
   VT *__restrict__ vdst = (VT *)((before & 1) ? vals0 : vals1);
 
   const int tid = threadIdx.x;
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63;
   const int bits = (hiBit - shift) < BITS ? (hiBit - shift) : BITS;
   const uint32_t dmask = (1u << bits) - 1u;
 
   if (tid == 0) s_tile = ticket(&st.tickets[pass]);
-  for (int i = tid; i < W * R; i += THREADS) (&s_whist[0][0])[i] = 0u;
+  for (int i = tid; i < W * R / 2; i += THREADS) ((uint32_t *)&s_whist[0][0])[i] = 0u;
   __syncthreads();
-  const uint32_t tile = s_tile;
+  const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
   const size_t tileBase = (size_t)tile * TILE;
   const size_t waveBase = tileBase + (size_t)w * (ITEMS * 64);
   const uint32_t valid = (n - tileBase) < (size_t)TILE ? (uint32_t)(n - tileBase) : (uint32_t)TILE;
 
   KT k[ITEMS];
-  uint32_t d[ITEMS];
-  uint32_t pos[ITEMS];
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    const size_t idx = waveBase + (size_t)j * 64 + l;
-    k[j] = idx < n ? src[idx] : ~(KT)0;
-    d[j] = digit_of(k[j], shift, dmask);
-  }
-  // The payloads are loaded with the keys, so their loads overlap the ranking and the look-back.
+  uint32_t pos[ITEMS / 2];  // two 16-bit positions each
+  const KT *__restrict__ wsrc = src + waveBase;
+  const VT *__restrict__ wvsrc = vsrc + (VB ? waveBase : 0);
+  const uint32_t here = valid > (uint32_t)w * (ITEMS * 64) ? valid - (uint32_t)w * (ITEMS * 64) : 0u;
+  load_items<ITEMS>(wsrc, valid == TILE, here, ~(KT)0, k);
+
+  // The payloads: in small workgroups loaded with the keys, which hides their latency best, in large
+  // ones once the keys are in LDS, when their registers are free.
+  constexpr bool kEarlyVals = VB != 0 && THREADS == 256;
   VT ve[VB ? ITEMS : 1];
-  if constexpr (VB != 0) {
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      const size_t idx = waveBase + (size_t)j * 64 + l;
-      ve[j] = idx < n ? vsrc[idx] : (VT)0;
-    }
-  }
+  if constexpr (kEarlyVals) load_items<ITEMS>(wvsrc, valid == TILE, here, (VT)0, ve);
 
   // Wave multisplit: peers with the same digit, rank among them, wave-private running counts.
 #pragma unroll
   for (int j = 0; j < ITEMS; ++j) {
-    const uint64_t m = match_digit<BITS>(d[j], ~0ull);
+    const uint32_t dj = digit_of(k[j], shift, dmask);
+    const uint64_t m = match_digit<BITS>(dj, ~0ull);
     const uint32_t r = mask_rank(m);
     const uint32_t c = (uint32_t)__popcll(m);
-    const uint32_t pre = s_whist[w][d[j]];
-    if (r == 0) s_whist[w][d[j]] = pre + c;
-    pos[j] = pre + r;
+    const uint32_t pre = s_whist[w][dj];
+    if (r == 0) s_whist[w][dj] = (uint16_t)(pre + c);
+    pos[j / 2] = j & 1 ? pos[j / 2] | (pre + r) << 16 : pre + r;
+    if constexpr (kTwoPerCU<KT, VB, THREADS>) {
+      asm volatile("" : "+v"(pos[j / 2]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
   __syncthreads();
 
@@ -241,7 +274,7 @@ __global__ void __launch_bounds__(THREADS)
 #pragma unroll
       for (int ww = 0; ww < W; ++ww) {
         const uint32_t c = s_whist[ww][dd];
-        s_whist[ww][dd] = sum;
+        s_whist[ww][dd] = (uint16_t)sum;
         sum += c;
       }
       cnt[q] = sum;
@@ -315,39 +348,58 @@ __global__ void __launch_bounds__(THREADS)
   KT *s_keys = (KT *)s_buf;
 #pragma unroll
   for (int j = 0; j < ITEMS; ++j) {
-    pos[j] = s_tdigit[d[j]] + s_whist[w][d[j]] + pos[j];
-    s_keys[pos[j]] = k[j];
+    if constexpr (kTwoPerCU<KT, VB, THREADS>) asm volatile("" : "+v"(k[j]));  // the digit is taken from the key again, not kept from the ranking
+    const uint32_t dj = digit_of(k[j], shift, dmask);
+    const uint32_t pj = s_tdigit[dj] + s_whist[w][dj] + (j & 1 ? pos[j / 2] >> 16 : pos[j / 2] & 0xFFFFu);
+    pos[j / 2] = j & 1 ? (pos[j / 2] & 0xFFFFu) | pj << 16 : (pos[j / 2] & 0xFFFF0000u) | pj;
+    s_keys[pj] = k[j];
+    if constexpr (kTwoPerCU<KT, VB, THREADS>) {
+      asm volatile("" : "+v"(pos[j / 2]));
+    }
   }
   __syncthreads();
 
+  if constexpr (VB != 0 && !kEarlyVals) load_items<ITEMS>(wvsrc, valid == TILE, here, (VT)0, ve);
   // The sorted keys back from LDS (every position of the tile holds a key, the padding included)
-  // and their global positions: all LDS reads are issued before the first write, so the wave waits
-  // once instead of twice per key.
-  KT sk[ITEMS];
-  uint32_t gaddr[ITEMS];
+  // and their global positions.
+  uint32_t dig[VB ? ITEMS / 4 : 1];  // the write positions' digits, a byte each
 #pragma unroll
-  for (int j = 0; j < ITEMS; ++j) sk[j] = s_keys[j * THREADS + tid];
+  for (int j0 = 0; j0 < ITEMS; j0 += NB) {
+    KT sk[NB];
 #pragma unroll
-  for (int j = 0; j < ITEMS; ++j) gaddr[j] = s_gbase[digit_of(sk[j], shift, dmask)] + (uint32_t)(j * THREADS + tid);
+    for (int j = 0; j < NB; ++j) sk[j] = s_keys[(j0 + j) * THREADS + tid];
 #pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    // gaddr < n always holds for the tile's own keys when histogram and look-back agree; it guards
-    // the write.
-    if ((uint32_t)(j * THREADS + tid) < valid && gaddr[j] < n) dst[gaddr[j]] = sk[j];
+    for (int j = 0; j < NB; ++j) {
+      const uint32_t dj = digit_of(sk[j], shift, dmask);
+      if constexpr (VB != 0) {
+        const int q = j0 + j;
+        dig[q / 4] = q & 3 ? dig[q / 4] | dj << 8 * (q & 3) : dj;
+      }
+      const uint32_t at = s_gbase[dj] + (uint32_t)((j0 + j) * THREADS + tid);
+      if ((uint32_t)((j0 + j) * THREADS + tid) < valid && at < n) put_at(dst, at, sk[j]);
+    }
+    if constexpr (kTwoPerCU<KT, VB, THREADS>) __builtin_amdgcn_sched_barrier(0);
   }
 
   if constexpr (VB != 0) {
     __syncthreads();
     VT *s_vals = (VT *)s_buf;
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) s_vals[pos[j]] = ve[j];
+    for (int j = 0; j < ITEMS; ++j) s_vals[j & 1 ? pos[j / 2] >> 16 : pos[j / 2] & 0xFFFFu] = ve[j];
     __syncthreads();
-    VT sv[ITEMS];
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j) sv[j] = s_vals[j * THREADS + tid];
+    for (int j0 = 0; j0 < ITEMS; j0 += NB) {
+      VT sv[NB];
 #pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-      if ((uint32_t)(j * THREADS + tid) < valid && gaddr[j] < n) vdst[gaddr[j]] = sv[j];
+      for (int j = 0; j < NB; ++j) sv[j] = s_vals[(j0 + j) * THREADS + tid];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int q = j0 + j;
+        const uint32_t at = s_gbase[(dig[q / 4] >> 8 * (q & 3)) & 255u] + (uint32_t)(q * THREADS + tid);
+        if ((uint32_t)((j0 + j) * THREADS + tid) < valid && at < n) put_at(vdst, at, sv[j]);
+      }
+      if constexpr (kTwoPerCU<KT, VB, THREADS>) __builtin_amdgcn_sched_barrier(0);
+    }
   }
 }
 
@@ -455,17 +507,15 @@ inline int passes_for(int loBit, int hiBit, int bits) { return (hiBit - loBit + 
 
 // Keys per tile of one sort. Automatically 2,048 (256 threads x 8) up to 2^18 keys, where a pass is as long
 // as one tile takes; 4,096 (256 x 16) for 64-bit keys or payloads and 8,192 (512 x 16) for narrow ones; and
-// 16,384 (1,024 x 16) from 1.5 million 64-bit keys, 2.6 million 64-bit payloads or 4 million narrow keys on,
-// where longer digit runs and fewer look-back steps count more. Us, with the smaller against the larger tile: 60,000 64-bit pairs 105 against 147, 260,000 134
-// against 173, 400,000 151 against 145; 60,000 32-bit pairs 66 against 79, 400,000 89 against 87; 1 million
-// 64-bit pairs 193 against 273, 4 million 439 against 362, 16 million 1508 against 1466, keys alone 176
-// against 200, 360 against 261, 944 against 749; 2 million pairs 270 against 301, keys 241 against 220. Asked for: 2,048, 4,096, and with narrow keys 8,192 and
-// 16,384 are taken as they are, with wide ones as 4,096.
-// (Payloads used to be loaded after the ranking where a key or payload has 64 bits: 16 million 64-bit pairs
-// 1775, now 1504 in tiles of the same size.)
+// 16,384 (1,024 x 16) from 1.6 million wide or 2.6 million narrow keys on, where longer digit runs and fewer
+// look-back steps count more. Us, with the smaller against the larger tile: 60,000 64-bit pairs 105 against
+// 147, 260,000 134 against 173, 400,000 151 against 145; 60,000 32-bit pairs 66 against 79, 400,000 89 against
+// 87; 1 million 64-bit pairs 194 against 242, 2 million 277 against 264, 64-bit keys 176 against 189 and 218
+// against 217; 2 million 32-bit pairs 124 against 129, 3 million 156 against 143. Asked for: 2,048, 4,096,
+// and with narrow keys 8,192 and 16,384 are taken as they are, with wide ones as 4,096.
 constexpr size_t kAutoSmallTileKeys = (size_t)1 << 18;
 constexpr size_t large_tile_keys(int keyBits, int valBits) {
-  return valBits == 64 ? (size_t)5 << 19 : keyBits == 64 ? (size_t)3 << 19 : (size_t)1 << 22;
+  return keyBits == 64 || valBits == 64 ? (size_t)3 << 19 : (size_t)5 << 19;
 }
 
 int tile_keys_effective(const SortConfig &cfg, size_t n, int keyBits, int valBits) {

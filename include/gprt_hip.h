@@ -293,7 +293,7 @@ GPRT_API uint32_t gprtBufferExclusiveSumNoAlloc(GPRTContext context, GPRTBuffer 
 /* Radix sort knobs used by every sort and accel build on this context (the autotuner's search
  * space): digitBits in {4, 6, 8}, tileKeys (keys per workgroup tile) in {2048, 4096, 8192, 16384}
  * or 0 (automatic: for accel builds 2048 to 16384 by the number of primitives and their mean per mesh;
- * for the buffer sorts 2048 up to 2^18 keys, 16384 from 1.5 to 4 million keys on by their size,
+ * for the buffer sorts 2048 up to 2^18 keys, 16384 from 1.6 or 2.6 million keys on by their size,
  * between them 4096 for 64-bit keys or payloads and 8192 for narrow ones; with 64-bit keys or
  * payloads 8192 and 16384 asked for count as 4096), wavesPerCU (0 = no cap) caps the resident waves of the accel
  * builds' sort passes through LDS padding (no effect at 16384 keys, whose 1024-thread tiles
