@@ -355,9 +355,8 @@ __global__ void __launch_bounds__(kTraceBlock)
   const LaneStack st{s_stack, tid, spill + (size_t)gtid * (kMaxStack - kLdsStack)};
   const int l = tid & 63;
   const bool more = count > gridDim.x * kTraceBlock;
-  bool first = true;
   do {
-    const uint32_t base = next_rays(work, first);
+    const uint32_t base = next_rays(work, more);
     if (base >= count) break;
     const uint32_t ri = base + (uint32_t)l;
     if (ri < count) {

@@ -44,9 +44,8 @@ __global__ void __launch_bounds__(kTraceBlock)
   const int l = tid & 63;
 
   const bool more = count > gridDim.x * kTraceBlock;
-  bool first = true;
   do {
-    const uint32_t base = next_rays(work, first);
+    const uint32_t base = next_rays(work, more);
     if (base >= count) break;
     const uint32_t ri = base + (uint32_t)l;
     if (ri < count) {
