@@ -65,23 +65,23 @@ LBVH_BYTES_PER_PRIM = 368
 # (FETCH_SIZE x 2.0 and WRITE_SIZE x 1.0, the factors a plain 1 GiB copy gives): read + write.
 # The commands and per-kernel tables are in profiles/hbm_bytes_build_trace.md.
 TRAFFIC_BYTES = {
-    "trace_closest": 28060.8e6 + 138.6e6,  # the plain trace of the workload's 8,388,608 rays
+    "trace_closest": 27292.9e6 + 237.8e6,  # the plain trace of the workload's 8,388,608 rays
     "mlp_infer_fused": 275.9e6 + 33.6e6,  # one launch of 8,388,608 rays, 2,897 classes bound
-    "lbvh_sort_pass": 30.9e6 + 35.3e6,  # one pass over 4,194,304 keys on 16,384-key tiles (mean of 4)
+    "lbvh_sort_pass": 30.8e6 + 35.5e6,  # one pass over 4,194,304 keys on 16,384-key tiles (mean of 4)
     # per primitive, summed over the build kernels (init, bounds, keys, histogram scan, 4 sort
     # passes, sub-tile, region, top)
     "build_per_prim": 0.3 + 60.1 + 16.2 + (4.4 + 8.6) + 3 * (8.4 + 8.4) + 263.8 + 1.1,
     "batched_build_per_prim": 0.7 + 60.1 + 16.5 + 0.1 + 4 * (7.61 + 9.18) + 220.1 + 1.4 + 0.04,
     "boxes_build_per_prim": 0.3 + 36.1 + 16.2 + (4.3 + 8.3) + 3 * (8.4 + 8.4) + 262.0 + 1.1,
     "refit_per_prim": 12.0 + 263.4 + 1.2,  # identity check, sub-tile (vertex gather), region + top
-    "trace_boxes": 14894.1e6 + 69.4e6,  # one launch of 4,194,304 rays
+    "trace_boxes": 15781.0e6 + 127.5e6,  # one launch of 4,194,304 rays
     "compute_bounds": 268.5e6 + 402.7e6,  # one launch over 16,777,216 spheres
-    "sort_onesweep": 556.5e6 + 566.3e6,  # one pass over 2^26 u32 keys + u32 payloads (16,384-key tiles)
+    "sort_onesweep": 568.9e6 + 584.8e6,  # one pass over 2^26 u32 keys + u32 payloads (16,384-key tiles)
     "scan_lookback": 1075.5e6 + 1078.1e6,  # one launch over 2^28 u32
 }
 # Vector L1 and L2 hit rates of the traversal kernel on this workload (rocprofv3 --pmc TCP_* / TCC_*;
 # commands and per-kernel table in profiles/cache_hit_rates_scene.md).
-TRACE_CACHE_HIT = {"l1": 0.807, "l2": 0.687}
+TRACE_CACHE_HIT = {"l1": 0.437, "l2": 0.720}
 
 
 def log(msg):

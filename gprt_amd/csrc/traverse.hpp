@@ -321,11 +321,11 @@ __device__ __forceinline__ bool slab_hit(const SlabRay &r, float lox, float loy,
 //
 // Times before and after, us, half primary and half bounce rays:
 //   through          512 rays     8,192       65,536      262,144     1,048,352    8,388,608
-//     16,384 tris   160 -> 40   185 -> 51   198 -> 69   226 -> 124    409 -> 277   2174 -> 1450
-//    262,144        270 -> 51   404 -> 70   443 -> 145  481 -> 326    941 -> 666   4844 -> 3400
-//  4,194,304        429 -> 62   584 -> 101  703 -> 226  811 -> 500   1610 -> 1134  7971 -> 5690
+//     16,384 tris   160 -> 40   185 -> 51   198 -> 69   226 -> 124    409 -> 271   2174 -> 1455
+//    262,144        270 -> 51   404 -> 70   443 -> 145  481 -> 326    941 -> 639   4844 -> 3309
+//  4,194,304        429 -> 62   584 -> 101  703 -> 226  811 -> 500   1610 -> 1041  7971 -> 5521
 // What bounds the largest now is the latency of the vector cache's misses (two thirds of the node fetches
-// miss L1, a third of those L2; the vector units are 58 % busy), the smallest the longest chain of nodes.
+// miss L1, a third of those L2; the vector units are 65 % busy), the smallest the longest chain of nodes.
 constexpr int kRefill = 12;
 constexpr int kSplitIdle = 24;
 constexpr uint32_t kSplitEvery = 2;
