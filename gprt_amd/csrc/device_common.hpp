@@ -87,4 +87,51 @@ __device__ __forceinline__ float ord2f(uint32_t u) {
   return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
 }
 
+// The rank of key `k` = keys[i0 + lane] among keys [0, n), ties by index, for a workgroup of 1,024 threads
+// (i0 a multiple of 64; the result is wave 0's). Its 16 waves share the comparisons with all keys, 128 bytes
+// at a time. Those are uniform over the wave and come through scalar loads, so a pair costs one compare and
+// one add with carry. The workgroup's own keys and the last few are compared from registers.
+template <typename KT>
+__device__ __forceinline__ KT read_lane(KT k, uint32_t lane) {
+  if constexpr (sizeof(KT) == 8)
+    return (KT)wave_read((uint32_t)(k >> 32), (int)lane) << 32 | wave_read((uint32_t)k, (int)lane);
+  else
+    return wave_read(k, (int)lane);
+}
+
+template <typename KT>
+__device__ __forceinline__ uint32_t key_rank(const KT *__restrict__ keys, uint32_t n, uint32_t i0, KT k,
+                                             uint32_t (&s_count)[16][64]) {
+  constexpr uint32_t W = 16, C = 128 / sizeof(KT);
+  const uint32_t l = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t chunks = n / C, own = i0 / C;
+  const KT tail = keys[min(chunks * C + l, n - 1)];
+  uint32_t count = 0;
+  for (uint32_t c = w; c < min(own, chunks); c += W) {
+#pragma unroll
+    for (uint32_t x = 0; x < C; ++x) count += keys[c * C + x] <= k ? 1u : 0u;
+  }
+  for (uint32_t c = own + 64u / C + w; c < chunks; c += W) {
+#pragma unroll
+    for (uint32_t x = 0; x < C; ++x) count += keys[c * C + x] < k ? 1u : 0u;
+  }
+  if (w == W - 1 && chunks * C >= i0 + 64u) {
+    for (uint32_t x = 0; x < n - chunks * C; ++x) count += read_lane(tail, x) < k ? 1u : 0u;
+  }
+#pragma unroll
+  for (uint32_t y = 0; y < 64u / W; ++y) {
+    const uint32_t x = w * (64u / W) + y;
+    const KT o = read_lane(k, x);
+    if (i0 + x < n) count += (o < k || (o == k && x < l)) ? 1u : 0u;
+  }
+  s_count[w][l] = count;
+  __syncthreads();
+  uint32_t rank = 0;
+  if (w == 0) {
+#pragma unroll
+    for (uint32_t x = 0; x < W; ++x) rank += s_count[x][l];
+  }
+  return rank;
+}
+
 }  // namespace gprt

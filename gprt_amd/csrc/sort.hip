@@ -425,56 +425,19 @@ __global__ void __launch_bounds__(256) k_final_copy(KT *__restrict__ keys0, cons
 // ------------------------------------------------------------------------------------------------
 // Small sorts: every key's rank by comparing it with every key.
 // ------------------------------------------------------------------------------------------------
-// One workgroup per 64 keys (lane = key); its 16 waves share the comparisons with all keys, 16 keys
-// at a time. Those are uniform over the wave and come through scalar loads, so a pair costs one compare
-// and one add with carry. The rank (ties by index: stable) is the key's place in `outKeys`. The
-// workgroup's own keys and the last n % 16 are compared from registers.
-template <typename KT>
-__device__ __forceinline__ KT read_lane(KT k, uint32_t lane) {
-  if constexpr (sizeof(KT) == 8)
-    return (KT)wave_read((uint32_t)(k >> 32), (int)lane) << 32 | wave_read((uint32_t)k, (int)lane);
-  else
-    return wave_read(k, (int)lane);
-}
-
+// One workgroup per 64 keys (key_rank): the rank is the key's place in `outKeys`.
 template <typename KT, int VB>
 __global__ void __launch_bounds__(1024)
     k_rank(const KT *__restrict__ keys, const void *__restrict__ vals, KT *__restrict__ outKeys,
            void *__restrict__ outVals, uint32_t n) {
   using VT = typename ValType<VB>::T;
-  constexpr uint32_t W = 16, C = 128 / sizeof(KT);
-  __shared__ uint32_t s_count[W][64];
-  const uint32_t l = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t i0 = blockIdx.x * 64u, i = min(i0 + l, n - 1);
+  __shared__ uint32_t s_count[16][64];
+  const uint32_t l = threadIdx.x & 63u, i0 = blockIdx.x * 64u, i = min(i0 + l, n - 1);
   const KT k = keys[i];
   VT v = 0;
-  if (VB && w == 0) v = ((const VT *)vals)[i];
-  const uint32_t chunks = n / C, own = i0 / C;
-  const KT tail = keys[min(chunks * C + l, n - 1)];
-  uint32_t count = 0;
-  for (uint32_t c = w; c < min(own, chunks); c += W) {
-#pragma unroll
-    for (uint32_t x = 0; x < C; ++x) count += keys[c * C + x] <= k ? 1u : 0u;
-  }
-  for (uint32_t c = own + 64u / C + w; c < chunks; c += W) {
-#pragma unroll
-    for (uint32_t x = 0; x < C; ++x) count += keys[c * C + x] < k ? 1u : 0u;
-  }
-  if (w == W - 1 && chunks * C >= i0 + 64u) {
-    for (uint32_t x = 0; x < n - chunks * C; ++x) count += read_lane(tail, x) < k ? 1u : 0u;
-  }
-#pragma unroll
-  for (uint32_t y = 0; y < 64u / W; ++y) {
-    const uint32_t x = w * (64u / W) + y;
-    const KT o = read_lane(k, x);
-    if (i0 + x < n) count += (o < k || (o == k && x < l)) ? 1u : 0u;
-  }
-  s_count[w][l] = count;
-  __syncthreads();
-  if (w == 0 && i0 + l < n) {
-    uint32_t rank = 0;
-#pragma unroll
-    for (uint32_t x = 0; x < W; ++x) rank += s_count[x][l];
+  if (VB && threadIdx.x < 64) v = ((const VT *)vals)[i];
+  const uint32_t rank = key_rank(keys, n, i0, k, s_count);
+  if (threadIdx.x < 64 && i0 + l < n) {
     outKeys[rank] = k;
     if (VB) ((VT *)outVals)[rank] = v;
   }

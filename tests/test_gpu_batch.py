@@ -179,3 +179,28 @@ def test_autotune_small_batch(ctx, orc):
         ctx.lib.gprtSetSortConfig(ctx.h, 8, 0, 0)
         for a in accs:
             a.destroy()
+
+
+@pytest.mark.parametrize("sizes", [[1], [15], [64], [65], [2047], [2049], [11585], [11586],
+                                   [1, 2, 3, 16, 17, 63, 64, 65, 128, 129, 2048, 4097]])
+def test_keys_by_ranks_equal_digit_passes(ctx, orc, sizes):
+    """Builds of few primitives sort their keys by ranks, unless a tile size is asked for: both give
+    the oracle's keys, nodes and boxes, with every third triangle a copy of the first (equal codes)."""
+    meshes = []
+    for k, n in enumerate(sizes):
+        v, idx = scenes.uniform_scene(n, seed=90 + n + k)
+        v = v.reshape(n, 3, 3).copy()
+        v[::3] = v[0]
+        meshes.append((v.reshape(-1, 3), idx))
+    try:
+        for tile in (0, 2048):
+            ctx.lib.gprtSetSortConfig(ctx.h, 8, tile, 0)
+            accs = [api.TriangleAccel(ctx, v, idx) for v, idx in meshes]
+            api.build_batch(ctx, accs)
+            assert api.last_error() is None, api.last_error()
+            for acc, (v, idx) in zip(accs, meshes):
+                _check(acc, orc, v, idx)
+            for a in accs:
+                a.destroy()
+    finally:
+        ctx.lib.gprtSetSortConfig(ctx.h, 8, 0, 0)
