@@ -421,15 +421,13 @@ __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_e
   __shared__ StreamLds lds;
   const uint32_t gtid = blockIdx.x * kTraceBlock + threadIdx.x;
   RayPre rw = {};
-  SlabRay slab = {};
   HitState h;
   hit_init(h, 0.0f);
   trace_stream(
-      topNodes, leaves, count, chunk, work, rw, slab, h, lds, spill + (size_t)gtid * (kMaxStack - kStreamStack),
+      topNodes, leaves, count, chunk, work, rw, h, lds, spill + (size_t)gtid * (kMaxStack - kStreamStack),
       [&](uint32_t ri) __attribute__((always_inline)) {
         const GPRTRay ray = load_ray_stream(rays + ri);
         rw = ray_setup(ray.ox, ray.oy, ray.oz, ray.tmin, ray.dx, ray.dy, ray.dz);
-        slab = slab_ray(rw);
         hit_init(h, ray.tmax);
       },
       [&](int pos) __attribute__((always_inline)) {

@@ -88,15 +88,13 @@ __global__ void __launch_bounds__(kTraceBlock)
   __shared__ StreamLds lds;
   const uint32_t gtid = blockIdx.x * kTraceBlock + threadIdx.x;
   RayPre r = {};
-  SlabRay slab = {};
   HitState h;
   hit_init(h, 0.0f);
   trace_stream(
-      nodes, nprims, count, chunk, work, r, slab, h, lds, spill + (size_t)gtid * (kMaxStack - kStreamStack),
+      nodes, nprims, count, chunk, work, r, h, lds, spill + (size_t)gtid * (kMaxStack - kStreamStack),
       [&](uint32_t ri) __attribute__((always_inline)) {
         const GPRTRay ray = load_ray_stream(rays + ri);
         r = ray_setup(ray.ox, ray.oy, ray.oz, ray.tmin, ray.dx, ray.dy, ray.dz);
-        slab = slab_ray(r);
         hit_init(h, ray.tmax);
       },
       [&](int pos) __attribute__((always_inline)) { intersect_leaf<kBoxes, true>(r, tris, pos, nprims, 0u, -1, h); },

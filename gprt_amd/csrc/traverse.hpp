@@ -244,54 +244,6 @@ __device__ __forceinline__ uint32_t traverse(const RayPre &r, const BVHNode *__r
   return walk_batched<MaxStack, decltype(leafTest) &>(r, nodes, nprims, start, h, st, sp0, skip, leafTest);
 }
 
-// A ray as the node test wants it. Per axis the distance to a plane p is p * i + b, b = -o * i: one FMA
-// instead of a subtraction and a multiplication. Its error beyond the relative ones (of i and of the
-// result, which the test's margin covers) is b's own rounding, at most 2^-24 |o * i|: the near plane's
-// b is lowered and the far plane's raised by twice that, which widens boxes by 2^-23 |o|, less than a
-// box's own coordinates near o are rounded. (One slack on the distances instead would let a ray with a
-// near-zero direction component, whose i is huge, enter every box.) Which plane is near follows from
-// the direction's sign, kept as lane masks. An axis whose products overflow is ignored.
-struct SlabRay {
-  float ix, iy, iz;  // reciprocal direction
-  float nx, ny, nz;  // b of the near planes
-  float fx, fy, fz;  // b of the far planes
-  float tmin;
-  bool px, py, pz;  // direction not negative: the near plane is the lower one
-};
-
-__device__ __forceinline__ void slab_axis(float o, float i, float &si, float &n, float &f, bool &p) {
-  const float b = -(o * i), e = fabsf(b) * 1.1920929e-07f;
-  const bool fine = fabsf(b) < 3.0e38f;
-  si = fine ? i : 0.0f;
-  n = fine ? b - e : -INFINITY;
-  f = fine ? b + e : INFINITY;
-  p = i >= 0.0f;
-}
-
-__device__ __forceinline__ SlabRay slab_ray(const RayPre &r) {
-  SlabRay s;
-  slab_axis(r.ox, r.ix, s.ix, s.nx, s.fx, s.px);
-  slab_axis(r.oy, r.iy, s.iy, s.ny, s.fy, s.py);
-  slab_axis(r.oz, r.iz, s.iz, s.nz, s.fz, s.pz);
-  s.tmin = r.tmin;
-  return s;
-}
-
-// Conservative test of a node's child box: accepted unless the later of its entry distance and tmin
-// exceeds the earlier of its exit distance and tbest by more than 2^-12 of the latter, far above the
-// rounding of the distances and of the primitive tests (the margin box_hit keeps). NaN distances are
-// ignored, so they accept. 18 vector instructions.
-__device__ __forceinline__ bool slab_hit(const SlabRay &r, float lox, float loy, float loz, float hix, float hiy,
-                                         float hiz, float tbest, float &tnear) {
-  const float nx = fmaf(r.px ? lox : hix, r.ix, r.nx), fx = fmaf(r.px ? hix : lox, r.ix, r.fx);
-  const float ny = fmaf(r.py ? loy : hiy, r.iy, r.ny), fy = fmaf(r.py ? hiy : loy, r.iy, r.fy);
-  const float nz = fmaf(r.pz ? loz : hiz, r.iz, r.nz), fz = fmaf(r.pz ? hiz : loz, r.iz, r.fz);
-  tnear = fmaxf(fmaxf(nx, ny), nz);
-  const float tf = fminf(fminf(fminf(fx, fy), fz), tbest);
-  return !(fmaxf(tnear, r.tmin) > fmaf(2.0f * kBoxSlack, fabsf(tf), tf));
-}
-
-
 // The plain trace: no proposal and no fetch counts. A wave keeps its 64 lanes busy. A lane whose ray has
 // ended gets the next one (with 64 fixed rays per wave, which walk until the longest one ends, 17 of 64
 // lanes are active on average), and once there is none left, a part of another lane's ray: the far subtree
@@ -321,11 +273,14 @@ __device__ __forceinline__ bool slab_hit(const SlabRay &r, float lox, float loy,
 //
 // Times before and after, us, half primary and half bounce rays:
 //   through          512 rays     8,192       65,536      262,144     1,048,352    8,388,608
-//     16,384 tris   160 -> 40   185 -> 51   198 -> 69   226 -> 124    409 -> 271   2174 -> 1455
-//    262,144        270 -> 51   404 -> 70   443 -> 145  481 -> 326    941 -> 639   4844 -> 3309
-//  4,194,304        429 -> 62   584 -> 101  703 -> 226  811 -> 500   1610 -> 1041  7971 -> 5521
+//     16,384 tris   160 -> 40   185 -> 51   198 -> 69   226 -> 124    409 -> 271   2174 -> 1503
+//    262,144        270 -> 51   404 -> 70   443 -> 145  481 -> 326    941 -> 639   4844 -> 3364
+//  4,194,304        429 -> 62   584 -> 101  703 -> 226  811 -> 500   1610 -> 1041  7971 -> 5571
 // What bounds the largest now is the latency of the vector cache's misses (two thirds of the node fetches
-// miss L1, a third of those L2; the vector units are 65 % busy), the smallest the longest chain of nodes.
+// miss L1, a third of those L2; the vector units are busy 70 % of the time), the smallest the longest chain of
+// nodes. The node test stays box_hit, as in every other walk: a test of 18 instead of 26 instructions (planes
+// by one FMA each, widened for its rounding) gained 1 % and found hits that box_hit does not enter, for rays
+// in the plane of a box's face.
 constexpr int kRefill = 12;
 constexpr int kSplitIdle = 24;
 constexpr uint32_t kSplitEvery = 2;
@@ -479,14 +434,14 @@ __device__ __forceinline__ void settle_parts(char *stage, int lane, int own, boo
   }
 }
 
-// Traces rays [0, count), `chunk` at a time: begin(i) sets up ray i in the caller's `ray`, `slab` and `h`,
+// Traces rays [0, count), `chunk` at a time: begin(i) sets up ray i in the caller's `ray` and `h`,
 // leaf(position) tests a leaf, end(i) stores ray i's hit. `work`: kShares counters, zeroed (read only if
 // there are more chunks than waves), kShareWords apart. `spill`: this lane's kMaxStack - kStreamStack
 // words. The tree has fewer than kSmallTreePrims primitives.
 template <class Begin, class Leaf, class End>
 __device__ __forceinline__ void trace_stream(const BVHNode *__restrict__ nodes, uint32_t nprims, uint32_t count,
-                                             uint32_t chunk, uint32_t *__restrict__ work, RayPre &ray, SlabRay &slab,
-                                             HitState &h, StreamLds &lds, uint32_t *__restrict__ spill, Begin &&begin,
+                                             uint32_t chunk, uint32_t *__restrict__ work, RayPre &ray, HitState &h,
+                                             StreamLds &lds, uint32_t *__restrict__ spill, Begin &&begin,
                                              Leaf &&leaf, End &&end) {
   constexpr uint32_t kDone = 0x80000000u, kNoRay = 0xFFFFFFFFu;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -583,7 +538,6 @@ __device__ __forceinline__ void trace_stream(const BVHNode *__restrict__ nodes, 
         const int theirOwn = from_lane(own, src);
         if (takes) {
           ray = theirs;
-          slab = slab_ray(ray);
           ri = theirRi;
           own = theirOwn;
           hit_init(h, best[own]);
@@ -613,8 +567,8 @@ __device__ __forceinline__ void trace_stream(const BVHNode *__restrict__ nodes, 
       float tn0, tn1, bound = h.t;
       if (!more) bound = fminf(bound, best[own]);
       // Lane masks rather than flags: they stay in scalar registers.
-      const uint64_t h0 = __ballot(slab_hit(slab, a.x, a.y, a.z, a.w, b.x, b.y, bound, tn0));
-      const uint64_t h1 = __ballot(slab_hit(slab, b.z, b.w, d.x, d.y, d.z, d.w, bound, tn1));
+      const uint64_t h0 = __ballot(box_hit(ray, a.x, a.y, a.z, a.w, b.x, b.y, bound, tn0));
+      const uint64_t h1 = __ballot(box_hit(ray, b.z, b.w, d.x, d.y, d.z, d.w, bound, tn1));
       const uint64_t n0 = __ballot(child.x >= 0), n1 = __ballot(child.y >= 0), near0 = __ballot(tn0 <= tn1);
       const uint64_t i0 = h0 & n0, i1 = h1 & n1, l0 = h0 & ~n0, l1 = h1 & ~n1;
       if (lane_of(l0 | l1)) {

@@ -335,3 +335,30 @@ def test_streamed_trace_equals_general_form(ctx, n, rays):
         b.destroy()
     tlas.destroy()
     acc.destroy()
+
+
+@pytest.mark.parametrize("offset", [0.0, 1000.0, 1e6])
+def test_streamed_trace_of_axis_parallel_rays(ctx, offset):
+    """Rays with zero, denormal and tiny direction components whose origins lie on vertex coordinates,
+    in the planes of boxes' faces: the plain trace enters the boxes that the general one enters."""
+    verts, idx = scenes.uniform_scene(20000, seed=9)
+    verts = (verts.astype(np.float64) + offset).astype(np.float32)
+    acc = _build(ctx, verts, idx)
+    r = scenes.random_rays(40000, seed=4)
+    for c in ("ox", "oy", "oz"):
+        r[c] = (r[c].astype(np.float64) + offset).astype(np.float32)
+    for k, c in enumerate(("dx", "dy", "dz")):
+        r[c][k::5] = 0.0
+    r["dx"][3::7], r["dy"][4::11], r["dz"][5::13] = 1e-38, -1e-31, 1e-30
+    on = verts[np.random.default_rng(5).integers(0, len(verts), len(r))]
+    r["ox"][::3], r["oy"][::3] = on[::3, 0], on[::3, 1]
+    n = len(r)
+    rb, vb = ctx.device_buffer(r), ctx.device_buffer(nbytes=4 * n)
+    h1, h2 = ctx.device_buffer(nbytes=16 * n), ctx.device_buffer(nbytes=16 * n)
+    api.trace_detail(ctx, acc, rb, h1, n)
+    api.trace_detail(ctx, acc, rb, h2, n, visits_buf=vb)
+    assert api.last_error() is None, api.last_error()
+    _assert_hits_equal(h1.read(api.HIT_DTYPE), h2.read(api.HIT_DTYPE))
+    for b in (rb, vb, h1, h2):
+        b.destroy()
+    acc.destroy()
