@@ -495,7 +495,7 @@ bool mlp_alloc(Context *ctx, Proposal *p, uint32_t maxBatch) {
   p->m = (float *)(b + oM);
   p->v = (float *)(b + oV);
   p->weights = MlpWeights{(uint16_t *)(b + oRows), (uint16_t *)(b + oFwd), (uint16_t *)(b + oBwd), (float *)(b + oBias)};
-  p->stats = (float *)(b + oStat);
+  p->stats = (TrainStats *)(b + oStat);
   p->X = (uint16_t *)(b + oX);
   p->H = (uint16_t *)(b + oH);
   p->Z = (float *)(b + oZ);

@@ -37,13 +37,19 @@ struct MlpWeights {
   float *bias;
 };
 
+// What an epoch has added up: the batches' mean losses, and the rays whose class was right.
+struct TrainStats {
+  double loss;
+  uint32_t correct, unused;
+};
+
 struct Proposal {
   void *block = nullptr;
   size_t blockBytes = 0;
   uint32_t maxBatch = 0;
   float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // fp32 params, grads, Adam moments
   MlpWeights weights{};
-  float *stats = nullptr;      // [0] loss sum, [1] correct count (as uint)
+  TrainStats *stats = nullptr;
   uint16_t *X = nullptr, *H = nullptr;  // features and hidden activations of gprtProposalLogits
   float *Z = nullptr;                   // its logits
   // A training batch: activations and their gradients, dZ (bf16 fragments), and the products' partial

@@ -338,7 +338,7 @@ GPRT_API void gprtProposalGradients(GPRTContext _ctx, GPRTProposal _p, GPRTBuffe
     return;
   }
   hipStream_t s = ctx->stream;
-  fill_u32(ctx, s, p->stats, 0u, 2);
+  fill_u32(ctx, s, p->stats, 0u, sizeof(TrainStats) / 4);
   mlp_gradients(ctx, s, p, rays->d, (const int32_t *)labels->d, count, count);
   hip_ok(hipMemcpyAsync(hostGrads, p->g, kMlpParams * 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(grads)");
   hipStreamSynchronize(s);
@@ -380,20 +380,18 @@ float train_core(Context *ctx, Proposal *p, const void *rays, const void *hits, 
   hipStreamSynchronize(s);
   float lastLoss = 0.f, acc = 0.f;
   for (uint32_t e = 0; e < epochs; ++e) {
-    fill_u32(ctx, s, p->stats, 0u, 2);
+    fill_u32(ctx, s, p->stats, 0u, sizeof(TrainStats) / 4);
     uint32_t batches = 0;
     for (uint32_t b0 = 0; b0 < labelled; b0 += p->maxBatch) {
       const uint32_t n = std::min<uint32_t>(p->maxBatch, labelled - b0);
       mlp_train_step(ctx, s, p, cRays + b0, cLabels + b0, n, lr);
       ++batches;
     }
-    float st[2];
-    hip_ok(hipMemcpyAsync(st, p->stats, 8, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(stats)");
+    TrainStats st{};
+    hip_ok(hipMemcpyAsync(&st, p->stats, sizeof(st), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(stats)");
     hipStreamSynchronize(s);
-    uint32_t correct;
-    std::memcpy(&correct, &st[1], 4);
-    lastLoss = batches ? st[0] / (float)batches : 0.f;
-    acc = labelled ? (float)correct / (float)labelled : 0.f;
+    lastLoss = batches ? (float)(st.loss / batches) : 0.f;
+    acc = labelled ? (float)st.correct / (float)labelled : 0.f;
   }
   if (accuracy) *accuracy = acc;
   return lastLoss;

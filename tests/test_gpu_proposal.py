@@ -487,3 +487,35 @@ def test_overlapped_proposal_trace(ctx, scene):
     for b in (rb, hb):
         b.destroy()
     prop.destroy()
+
+
+def test_epoch_loss_and_accuracy(ctx):
+    """The mean loss and the accuracy of an epoch of half a million rays against 64 bits: one batch again
+    and again at a learning rate of 0, and a ragged last one, whose mean counts like the others'.
+
+    The bound: a row's sum of exponentials is off by at most 35 x 2^-24 of itself (expf 2 ulp, its argument
+    below 16 rounded once, 23 additions), its logarithm below 16 by 2 ulp (2^-19), the two additions by 2^-21
+    (below 16) and 2^-20 (below 32), and the mean is rounded to fp32 (2^-21): 5.9e-6. The sum over the rays
+    may add nothing to that; one running fp32 sum adds 1e-4 and more."""
+    batch, last, batches = 1024, 300, 512
+    prop = api.Proposal(ctx, max_batch=batch, seed=8)
+    rays = scenes.random_rays(batch, seed=8)
+    z = _logits(ctx, prop, rays).astype(np.float64)
+    top = z.argmax(1)
+    assert (z.max(1) - z.min(1)).max() < 16
+    labels = np.random.default_rng(8).integers(0, 4096, batch).astype(np.int32)
+    labels[::3] = top[::3]
+    peak = z.max(1)
+    row = np.log(np.exp(z - peak[:, None]).sum(1)) + peak - z[np.arange(batch), labels]
+    assert row.max() < 32
+    n = (batches - 1) * batch + last
+    rb = ctx.device_buffer(np.tile(rays, batches)[:n])
+    lb = ctx.device_buffer(np.tile(labels, batches)[:n])
+    loss, accuracy = prop.train_labels(rb, lb, n, epochs=1, lr=0.0)
+    assert api.last_error() is None, api.last_error()
+    assert abs(loss - ((batches - 1) * row.mean() + row[:last].mean()) / batches) <= 6e-6
+    right = labels == top
+    assert accuracy == np.float32((batches - 1) * int(right.sum()) + int(right[:last].sum())) / np.float32(n)
+    rb.destroy()
+    lb.destroy()
+    prop.destroy()
