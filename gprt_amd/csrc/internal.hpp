@@ -10,6 +10,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -94,6 +95,9 @@ struct Context {
   // Trace work counter (first 256 B) and per-lane stack spill area.
   void *traceScratch = nullptr;
   size_t traceBytes = 0;
+  // A scan call of any thread holds the lock from taking its epoch and sequence number until it has read
+  // its total: state and host word are one per context, and the stream runs the scans one by one anyway.
+  std::mutex scanMutex;
   // Pinned host word {sequence | total} that the scan kernels write, its device address, and the
   // number of the call that wrote it last.
   uint64_t *pinnedWord = nullptr, *pinnedWordDev = nullptr;

@@ -435,7 +435,7 @@ GPRT_API void gprtBufferCopy(GPRTContext _ctx, GPRTBuffer _src, GPRTBuffer _dst,
 // Scan family (gprt/gprt.cpp:8739-8818)
 // ------------------------------------------------------------------------------------------------
 // The total of call `seq`, once its output is complete. A scan that signals (one tile) is waited for by
-// watching the host word for a while, which takes half the time of an event's round trip.
+// watching the host word for a while, which takes half the time of an event's round trip. Under scanMutex.
 static uint32_t scan_total(Context *ctx, uint32_t seq, bool signals, const char *fn) {
   volatile uint64_t *const word = ctx->pinnedWord;
   if (signals) {
@@ -478,14 +478,11 @@ static uint32_t buffer_scan(GPRTContext _ctx, GPRTBuffer _in, GPRTBuffer _out, G
     fail("%s: %zu items exceeds the 32-bit item count", fn, n);
     return (uint32_t)-1;
   }
-  if (scratch) {
-    if (scratch->kind == BufKind::Host) {
-      fail("%s: scratch must be a device buffer", fn);
-      return (uint32_t)-1;
-    }
-    const size_t need = scan_scratch_bytes(n);  // an undersized scratch is resized, as documented
-    if (scratch->size < need && !buffer_realloc(scratch, need, false)) return (uint32_t)-1;
+  if (scratch && scratch->kind == BufKind::Host) {
+    fail("%s: scratch must be a device buffer", fn);
+    return (uint32_t)-1;
   }
+  std::lock_guard<std::mutex> lock(ctx->scanMutex);
   const uint32_t seq = ++ctx->scanSeq;
   if (!scan_run_kept(ctx, ctx->stream, (const uint32_t *)in->d, (uint32_t *)out->d, n, mode, selectPositive,
                      ctx->pinnedWordDev, seq))
@@ -522,6 +519,7 @@ GPRT_API uint32_t gprtBufferExclusiveSumNoAlloc(GPRTContext _ctx, GPRTBuffer _in
     fail("%s: no static scan state on device %d", fn, ctx->device);
     return (uint32_t)-1;
   }
+  std::lock_guard<std::mutex> lock(ctx->scanMutex);
   const uint32_t seq = ++ctx->scanSeq;
   scan_run(ctx, ctx->stream, (const uint32_t *)in->d, (uint32_t *)out->d, n, 0, false, state, ctx->pinnedWordDev, seq);
   return scan_total(ctx, seq, scan_signals(n, 0), fn);

@@ -112,8 +112,10 @@ GPRT_API void gprtBufferCopy(GPRTContext context, GPRTBuffer src, GPRTBuffer dst
  * total. Partition places selected items first in input order and unselected items at the tail
  * in reverse order (gprt/gprt_scan.slang:89-92); Select compacts the selected items. Selection
  * is "v >= 0" when selectPositive, else "v < 0" (tests/t03-bufferScans/hostCode.cpp:117).
- * scratch may be null (internal allocation) or undersized (resized in place), as documented at
- * gprt/gprt_host.h:2238-2241. The return value requires a host wait (the reference maps scratch).
+ * scratch (gprt/gprt_host.h:2238-2241) may be null or of any size and is neither used nor resized: the
+ * look-back state is the context's own (8 bytes per 4,096 to 45,056 items, allocated on first use). The
+ * return value requires a host wait (the reference maps scratch). Calls of several host threads on one
+ * context run one after another.
  * ------------------------------------------------------------------------------------------- */
 GPRT_API uint32_t gprtBufferExclusiveSum(GPRTContext context, GPRTBuffer input, GPRTBuffer output,
                                          GPRTBuffer scratch GPRT_IF_CPP(= nullptr));

@@ -6,6 +6,7 @@ hostCode.cpp: key-only random keys, key-value with unique shuffled keys), plus s
 wrap-around, edge sizes and the full-size microbenchmarks. Bar: bit-exact.
 """
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -120,6 +121,48 @@ def test_scan_family_tiles(ctx, n):
     assert total == int(c[-1]) & 0xFFFFFFFF
     assert out[0] == 0
     np.testing.assert_array_equal(out[1:], (c[:-1] & np.uint64(0xFFFFFFFF)).astype(np.uint32))
+
+
+def test_scans_of_several_threads(ctx):
+    """Scans of four host threads on one context, each with buffers and scratch of its own, over sizes
+    that grow (and with them the context's look-back state): every output and total is that call's own."""
+    sizes = [1000, 4097, 70_001, 16_384, 200_003, 1_000_003, 50_000, 7_000_001]
+
+    def prepare(t):
+        calls = []
+        for i, n in enumerate(sizes):
+            x = np.random.default_rng(100 * t + i).integers(-2**31, 2**31, n + t, dtype=np.int64).astype(np.int32)
+            calls.append((x, ctx.device_buffer(x), [ctx.device_buffer(nbytes=x.nbytes) for _ in range(3)]))
+        return calls, ctx.device_buffer(nbytes=4)
+
+    def go(work, totals):
+        calls, scratch = work
+        for _, inp, out in calls:
+            for _ in range(4):
+                totals.append((ctx.lib.gprtBufferExclusiveSum(ctx.h, inp.h, out[0].h, scratch.h),
+                               ctx.lib.gprtBufferPartition(ctx.h, inp.h, True, out[1].h, scratch.h),
+                               ctx.lib.gprtBufferExclusiveSumNoAlloc(ctx.h, inp.h, out[2].h)))
+
+    work = [prepare(t) for t in range(4)]
+    totals = [[] for _ in work]
+    threads = [threading.Thread(target=go, args=a) for a in zip(work, totals)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert api.last_error() is None, api.last_error()
+    for (calls, scratch), got in zip(work, totals):
+        for i, (x, inp, out) in enumerate(calls):
+            c = np.cumsum(x.view(np.uint32), dtype=np.uint64).astype(np.uint32)
+            sel = x[x >= 0]
+            assert got[4 * i:4 * i + 4] == [(int(c[-1]), len(sel), int(c[-1]))] * 4
+            for o in (out[0], out[2]):
+                np.testing.assert_array_equal(o.read(np.uint32)[1:], c[:-1])
+            np.testing.assert_array_equal(out[1].read(np.int32), np.concatenate([sel, x[x < 0][::-1]]))
+            for b in [inp] + out:
+                b.destroy()
+        assert scratch.nbytes == 4  # not used, not resized
+        scratch.destroy()
 
 
 def test_exclusive_sum_full_size(ctx):
