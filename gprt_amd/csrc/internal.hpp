@@ -186,7 +186,7 @@ struct BVHStore {
   uint32_t meshes = 0, prims = 0, inner = 0, tiles = 0;
   uint32_t primCap = 0, meshCap = 0, tileCap = 0;
   SortConfig cfg;    // tile size / digit width the arrays were laid out for
-  bool ranks = false;  // keys sorted by ranks instead of the digit passes
+  uint32_t ranks = 0;  // keys sorted by ranks, with so many workgroups per tile (0: by the digit passes)
   int passes = 0;
   void *block = nullptr;
   size_t blockBytes = 0;

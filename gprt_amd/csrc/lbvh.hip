@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "build_rule.hpp"
 #include "bvh.hpp"
 #include "device_common.hpp"
 #include "internal.hpp"
@@ -1372,7 +1373,7 @@ BuildArgs args_of(BVHStore *st) {
   a.ids = st->ids;
   a.codesTmp = st->codesTmp;
   a.idsTmp = st->idsTmp;
-  a.ranks = st->ranks ? 1u : 0u;
+  a.ranks = st->ranks;
   a.keysOut = st->ranks ? st->codesTmp : st->codes;
   a.nodes = (BVHNode *)st->nodes;
   a.tris = (TriRecord *)st->tris;
@@ -1430,8 +1431,7 @@ size_t sort_lds_pad(int wavesPerCU) {
 template <int BITS>
 void launch_sort(Context *ctx, hipStream_t s, BVHStore *st, const BuildArgs &a) {
   if (st->ranks) {
-    const uint32_t perTile = (uint32_t)st->cfg.tileKeys / 64;
-    launch(ctx, s, "lbvh_sort_ranks", k_rank, dim3(st->tiles * perTile), dim3(1024), 0, a, perTile);
+    launch(ctx, s, "lbvh_sort_ranks", k_rank, dim3(st->tiles * st->ranks), dim3(1024), 0, a, st->ranks);
     return;
   }
   launch(ctx, s, "lbvh_hist_scan", k_hist_scan<BITS>, dim3(st->meshes), dim3(256), 0, a);
@@ -1479,7 +1479,7 @@ void enqueue_build(Context *ctx, hipStream_t s, BVHStore *st) {
   launch_refit(ctx, s, st, a, 0u, st->tiles, 0u, st->meshes, true);
 }
 
-bool same_plan(const BVHStore *st, const std::vector<MeshDesc> &desc, const SortConfig &cfg, bool ranks) {
+bool same_plan(const BVHStore *st, const std::vector<MeshDesc> &desc, const SortConfig &cfg, uint32_t ranks) {
   if (st->ranks != ranks) return false;
   if (st->cfg.digitBits != cfg.digitBits || st->cfg.tileKeys != cfg.tileKeys || st->cfg.wavesPerCU != cfg.wavesPerCU)
     return false;
@@ -1500,7 +1500,7 @@ void free_block(BVHStore *st) {
 
 // Lays the arrays of `st` out for the given plan (reusing the allocation when it is big enough).
 bool store_layout(BVHStore *st, const std::vector<MeshDesc> &desc, const std::vector<uint32_t> &tileMesh,
-                  const SortConfig &cfg, bool ranks, uint32_t prims) {
+                  const SortConfig &cfg, uint32_t ranks, uint32_t prims) {
   const uint32_t M = (uint32_t)desc.size(), T = (uint32_t)tileMesh.size();
   const uint32_t I = prims - M;  // every mesh has ntri - 1 inner nodes
   const int R = 1 << cfg.digitBits;
@@ -1668,21 +1668,10 @@ static int auto_tile_keys(Accel **accels, uint32_t count) {
   return mean < 5u << 19 ? 8192 : 16384;
 }
 
-// Whether the keys are sorted by ranks (with the automatic configuration): up to 2^27 comparisons, one mesh
-// of 11,585 primitives. A build, us, by the digit passes and by ranks: 500 triangles 62 / 43, 2,000 74 / 59,
-// 5,000 85 / 67, 10,000 88 / 79, 16,384 93 / 92, 20,000 92 / 130; 16 meshes of up to 4,096 92 / 77, 300 of them
-// 191 / 275.
-static bool sort_by_ranks(Accel **accels, uint32_t count) {
-  uint64_t pairs = 0;
-  for (uint32_t m = 0; m < count; ++m) pairs += (uint64_t)accels[m]->geom->icount * accels[m]->geom->icount;
-  return pairs <= 1ull << 27;
-}
-
 bool lbvh_build_batch(Context *ctx, hipStream_t s, Accel **accels, uint32_t count, bool useGraph,
                       bool layoutOnly) {
   SortConfig cfg = ctx->sortCfg;
   if (cfg.tileKeys == 0) cfg.tileKeys = auto_tile_keys(accels, count);
-  const bool ranks = ctx->sortCfg.tileKeys == 0 && sort_by_ranks(accels, count);
   const uint32_t tileKeys = (uint32_t)cfg.tileKeys;
   std::vector<MeshDesc> desc(count);
   std::vector<uint32_t> tileMesh;
@@ -1703,6 +1692,8 @@ bool lbvh_build_batch(Context *ctx, hipStream_t s, Accel **accels, uint32_t coun
     fail("gprtAccelBuild: %llu triangles in one build exceeds the 2^30 limit", (unsigned long long)prims);
     return false;
   }
+  const uint32_t ranks =
+      ctx->sortCfg.tileKeys == 0 ? rank_groups(count, tileKeys, [&](uint32_t m) { return desc[m].ntri; }) : 0u;
   tileMesh.resize(tiles);
   for (uint32_t m = 0; m < count; ++m)
     for (uint32_t t = 0; t < desc[m].ntiles; ++t) tileMesh[desc[m].tileOffset + t] = m;

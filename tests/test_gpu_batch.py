@@ -204,3 +204,22 @@ def test_keys_by_ranks_equal_digit_passes(ctx, orc, sizes):
                 a.destroy()
     finally:
         ctx.lib.gprtSetSortConfig(ctx.h, 8, 0, 0)
+
+
+@pytest.mark.parametrize("sizes", [[64] * 700, [3] * 500 + [130], [600] + [64] * 900, [2000] + [8] * 500,
+                                   [2000] + [8] * 1000, [1, 63, 65, 2049] + [17] * 600])
+def test_batches_of_many_small_meshes(ctx, orc, sizes):
+    """Batches on either side of the rule that bounds the idle workgroups of the sort by ranks give the
+    oracle's keys, nodes and boxes (the larger meshes and every 50th)."""
+    meshes = []
+    for k, n in enumerate(sizes):
+        v, idx = scenes.uniform_scene(n, seed=7 + k)
+        meshes.append((v, idx))
+    accs = [api.TriangleAccel(ctx, v, idx) for v, idx in meshes]
+    api.build_batch(ctx, accs)
+    assert api.last_error() is None, api.last_error()
+    for k, (acc, (v, idx)) in enumerate(zip(accs, meshes)):
+        if k % 50 == 0 or k < 4 or k == len(accs) - 1:
+            _check(acc, orc, v, idx)
+    for a in accs:
+        a.destroy()
