@@ -1652,26 +1652,10 @@ void accel_detach(Accel *a) {
   }
 }
 
-// The automatic tile size. Bounds, keys and sort passes run one workgroup per tile, so few primitives
-// want small tiles, that every CU gets one, and batches of small meshes, that their tiles are not mostly
-// empty; large meshes want large ones, for fewer look-back steps. One mesh of n triangles, us, with tiles of
-// 2,048 / 4,096 / 8,192 / 16,384: 16,384: 92 / 104 / 118 / 138, 200,000: 126 / 135 / 148 / 185, 500,000:
-// 159 / 157 / 168 / 198, 1 million: 236 / 212 / 205 / 237, 2 million: 367 / 317 / 288 / 314, 3 million: 501 /
-// 429 / 399 / 388. A thousand meshes of 970 on average: 421 / 468 / 607 / 914, of 9,400: 1372 / 1285 / 1387 /
-// 1687; 64 of 65,536 with their top level: 2594 / 2433 / 2323 / 2281.
-static int auto_tile_keys(Accel **accels, uint32_t count) {
-  uint64_t prims = 0;
-  for (uint32_t m = 0; m < count; ++m) prims += accels[m]->geom->icount;
-  const uint64_t mean = prims / count;
-  if (prims <= 384u << 10 || mean < 2048) return 2048;
-  if (prims <= 768u << 10 || mean < 16384) return 4096;
-  return mean < 5u << 19 ? 8192 : 16384;
-}
-
 bool lbvh_build_batch(Context *ctx, hipStream_t s, Accel **accels, uint32_t count, bool useGraph,
                       bool layoutOnly) {
   SortConfig cfg = ctx->sortCfg;
-  if (cfg.tileKeys == 0) cfg.tileKeys = auto_tile_keys(accels, count);
+  if (cfg.tileKeys == 0) cfg.tileKeys = auto_tile_keys(count, [&](uint32_t m) { return accels[m]->geom->icount; });
   const uint32_t tileKeys = (uint32_t)cfg.tileKeys;
   std::vector<MeshDesc> desc(count);
   std::vector<uint32_t> tileMesh;

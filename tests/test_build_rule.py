@@ -1,4 +1,4 @@
-"""The rule that picks the sort of a build's keys (gprt_amd/csrc/build_rule.hpp), compiled and asked on the host."""
+"""The rules that pick tile size and sort of a build's keys (gprt_amd/csrc/build_rule.hpp), compiled and asked on the host."""
 import os
 import subprocess
 
@@ -10,12 +10,14 @@ PROGRAM = """
 #include <cstdio>
 #include <vector>
 #include "gprt_amd/csrc/build_rule.hpp"
-int main() {  // lines of: tile size, number of {meshes, primitives} pairs, the pairs
+int main() {  // lines of: tile size (0: asks for it), number of {meshes, primitives} pairs, the pairs
   unsigned tile, parts;
   while (std::scanf("%u %u", &tile, &parts) == 2) {
     std::vector<unsigned> sizes;
     for (unsigned p = 0, count, n; p < parts && std::scanf("%u %u", &count, &n) == 2; ++p) sizes.insert(sizes.end(), count, n);
-    std::printf("%u\\n", gprt::rank_groups((unsigned)sizes.size(), tile, [&](unsigned m) { return sizes[m]; }));
+    auto size = [&](unsigned m) { return sizes[m]; };
+    const unsigned meshes = (unsigned)sizes.size();
+    std::printf("%u\\n", tile ? gprt::rank_groups(meshes, tile, size) : (unsigned)gprt::auto_tile_keys(meshes, size));
   }
 }
 """
@@ -56,3 +58,12 @@ def test_which_builds_take_ranks(rule):
     assert rule([(4096, 64)]) == 1 and rule([(1000, 8), (1, 150)]) == 3
     assert rule([(1, 2000), (500, 8)]) == 32 and rule([(1, 2000), (1000, 8)]) == 0
     assert rule([(65536, 8)]) == 1 and rule([(3_000_000, 4)]) == 0
+
+
+def test_tile_sizes(rule):
+    """Many meshes of a little over 12,288 primitives take two tiles of 8,192 each rather than four of 4,096."""
+    assert rule([(300, 12288)], 0) == 4096 and rule([(300, 12289)], 0) == 8192 and rule([(300, 15000)], 0) == 8192
+    assert rule([(1, 384 << 10)], 0) == 2048 and rule([(1, (384 << 10) + 1)], 0) == 4096
+    assert rule([(1, 768 << 10)], 0) == 4096 and rule([(1, (768 << 10) + 1)], 0) == 8192
+    assert rule([(1, (5 << 19) - 1)], 0) == 8192 and rule([(1, 5 << 19)], 0) == 16384
+    assert rule([(4000, 50), (1, 4_000_000)], 0) == 2048
