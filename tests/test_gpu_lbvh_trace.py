@@ -362,3 +362,69 @@ def test_streamed_trace_of_axis_parallel_rays(ctx, offset):
     for b in (rb, vb, h1, h2):
         b.destroy()
     acc.destroy()
+
+
+def _both_forms(ctx, acc, rays):
+    """Hits and instances of the streamed and the general trace, which must agree bit for bit; the hits."""
+    n = len(rays)
+    rb, vb = ctx.device_buffer(rays), ctx.device_buffer(nbytes=4 * n)
+    h1, h2 = ctx.device_buffer(nbytes=16 * n), ctx.device_buffer(nbytes=16 * n)
+    i1, i2 = ctx.device_buffer(nbytes=4 * n), ctx.device_buffer(nbytes=4 * n)
+    api.trace_detail(ctx, acc, rb, h1, n, i1)
+    api.trace_detail(ctx, acc, rb, h2, n, i2, visits_buf=vb)
+    assert api.last_error() is None, api.last_error()
+    hits = h1.read(api.HIT_DTYPE)
+    _assert_hits_equal(hits, h2.read(api.HIT_DTYPE))
+    np.testing.assert_array_equal(i1.read(np.int32), i2.read(np.int32))
+    for b in (rb, vb, h1, h2, i1, i2):
+        b.destroy()
+    return hits
+
+
+@pytest.mark.parametrize("rays", [350_000, 700_001])
+@pytest.mark.parametrize("kind", ["triangles", "boxes", "instances"])
+def test_streamed_trace_of_large_trees(ctx, kind, rays):
+    """Trees of 65,536 primitives and more, and more than 64 rays for each wave of a full launch: chunks of
+    32 rays, taken from the shares' counters. Every triangle twice, so that parts of a split ray end in ties;
+    random rays and the coherent ones of a pinhole camera, of which enough hit."""
+    verts, idx = scenes.uniform_scene(40_000, seed=31)
+    idx = np.ascontiguousarray(np.concatenate([idx, idx]))
+    acc = _build(ctx, verts, idx)
+    made = [acc]
+    if kind == "boxes":
+        corners = verts[idx]
+        made.append(api.AABBAccel(ctx, np.concatenate([corners.min(1), corners.max(1)], 1).astype(np.float32)))
+        made[-1].build()
+    elif kind == "instances":
+        moved = np.eye(3, 4, dtype=np.float32)
+        moved[:, 3] = np.float32(0.05)
+        made.append(api.InstanceAccel(ctx, api.instance_records([acc, acc], transforms=[np.eye(3, 4, dtype=np.float32), moved])))
+        made[-1].build()
+    wide = 700
+    for r in (scenes.random_rays(rays, seed=rays), scenes.pinhole_rays(wide, -(-rays // wide))[:rays]):
+        hits = _both_forms(ctx, made[-1], np.ascontiguousarray(r))
+        assert (hits["primID"] >= 0).mean() > 0.02
+    for a in reversed(made):
+        a.destroy()
+
+
+@pytest.mark.parametrize("offset,scale", [(0.0, 1.0), (1000.0, 10.0), (1e6, 1e3)])
+def test_streamed_trace_of_axis_parallel_rays_that_hit(ctx, offset, scale):
+    """As test_streamed_trace_of_axis_parallel_rays, with scenes that grow with their distance from the
+    origin, so that no triangle collapses to a point there, and a floor on the hits."""
+    verts, idx = scenes.uniform_scene(20000, seed=9)
+    verts = (verts.astype(np.float64) * scale + offset).astype(np.float32)
+    r = scenes.random_rays(40000, seed=4)
+    for c in ("ox", "oy", "oz"):
+        r[c] = (r[c].astype(np.float64) * scale + offset).astype(np.float32)
+    for k, c in enumerate(("dx", "dy", "dz")):
+        r[c][k::5] = 0.0
+    r["dx"][3::7], r["dy"][4::11], r["dz"][5::13] = 1e-38, -1e-31, 1e-30
+    on = verts[np.random.default_rng(5).integers(0, len(verts), len(r))]
+    r["ox"][::3], r["oy"][::3] = on[::3, 0], on[::3, 1]
+    corners = verts[idx].astype(np.float64)
+    assert (np.linalg.norm(np.cross(corners[:, 1] - corners[:, 0], corners[:, 2] - corners[:, 0]), axis=1) > 0).all()
+    acc = _build(ctx, verts, idx)
+    hits = _both_forms(ctx, acc, r)
+    assert (hits["primID"] >= 0).mean() > 0.05
+    acc.destroy()
