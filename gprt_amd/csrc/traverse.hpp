@@ -276,9 +276,14 @@ __device__ __forceinline__ uint32_t traverse(const RayPre &r, const BVHNode *__r
 //     16,384 tris   160 -> 40   185 -> 51   198 -> 69   226 -> 124    409 -> 271   2174 -> 1503
 //    262,144        270 -> 51   404 -> 70   443 -> 145  481 -> 326    941 -> 639   4844 -> 3364
 //  4,194,304        429 -> 62   584 -> 101  703 -> 226  811 -> 500   1610 -> 1041  7971 -> 5571
-// What bounds the largest now is the latency of the vector cache's misses (two thirds of the node fetches
-// miss L1, a third of those L2; the vector units are busy 70 % of the time), the smallest the longest chain of
-// nodes. The node test stays box_hit, as in every other walk: a test of 18 instead of 26 instructions (planes
+// What bounds the largest now is what the vector cache misses: 56 % of its accesses, 28 % of those L2 too, for
+// 27.5 GB of which the bounce half takes 26 (6.2 KB a ray); the smallest the longest chain of nodes. Only very
+// many coherent rays were faster with one ray per lane, as their waves stay together by themselves: 8 million
+// primary rays through 4 instances of 60,000 triangles 2,270 -> 2,580, 16 of 20,000 2,650 -> 2,990, through
+// 60,000 triangles 1,720 -> 1,860, 240,000 2,550 -> 2,800 (their bounce rays 6,450 -> 3,880; 20,000 triangles
+// 1,555 -> 1,330, a million 3,930 -> 3,880). The host cannot tell them from others. Handing rays out only to a
+// whole free wave gave 0 to 9 % of it back and doubled the bounce rays' time, a node that all lanes share loaded
+// without LDS cost all traces 2 to 10 %. The node test stays box_hit, as in every other walk: a test of 18 instead of 26 instructions (planes
 // by one FMA each, widened for its rounding) gained 1 % and found hits that box_hit does not enter, for rays
 // in the plane of a box's face.
 constexpr int kRefill = 12;

@@ -297,7 +297,9 @@ GPRT_API uint32_t gprtBufferExclusiveSumNoAlloc(GPRTContext context, GPRTBuffer 
  * or 0 (automatic: for accel builds 2048 to 16384 by the number of primitives and their mean per mesh;
  * for the buffer sorts 2048 up to 2^18 keys, 16384 from 1.6 or 2.6 million keys on by their size,
  * between them 4096 for 64-bit keys or payloads and 8192 for narrow ones; with 64-bit keys or
- * payloads 8192 and 16384 asked for count as 4096), wavesPerCU (0 = no cap) caps the resident waves of the accel
+ * payloads 8192 and 16384 asked for count as 4096). They are knobs of the digit passes: buffer sorts of up
+ * to 16384 keys, whatever is asked, and with tileKeys 0 accel builds of few primitives (one mesh of up to
+ * 11585) place each key by comparing it with the others instead. wavesPerCU (0 = no cap) caps the resident waves of the accel
  * builds' sort passes through LDS padding (no effect at 16384 keys, whose 1024-thread tiles
  * already run one per CU). Results do not depend on them. Default: 8, 0, 0. */
 GPRT_API void gprtSetSortConfig(GPRTContext context, uint32_t digitBits, uint32_t tileKeys, uint32_t wavesPerCU);
