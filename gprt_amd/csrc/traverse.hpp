@@ -282,10 +282,11 @@ __device__ __forceinline__ uint32_t traverse(const RayPre &r, const BVHNode *__r
 // primary rays through 4 instances of 60,000 triangles 2,270 -> 2,580, 16 of 20,000 2,650 -> 2,990, through
 // 60,000 triangles 1,720 -> 1,860, 240,000 2,550 -> 2,800 (their bounce rays 6,450 -> 3,880; 20,000 triangles
 // 1,555 -> 1,330, a million 3,930 -> 3,880). The host cannot tell them from others. Handing rays out only to a
-// whole free wave gave 0 to 9 % of it back and doubled the bounce rays' time, a node that all lanes share loaded
-// without LDS cost all traces 2 to 10 %. The node test stays box_hit, as in every other walk: a test of 18 instead of 26 instructions (planes
-// by one FMA each, widened for its rounding) gained 1 % and found hits that box_hit does not enter, for rays
-// in the plane of a box's face.
+// whole free wave gave 0 to 9 % of it back and doubled the bounce rays' time; a node that all lanes share,
+// loaded without LDS, cost all traces 2 to 10 %.
+// The node test stays box_hit, as in every other walk: a test of 18 instead of 26 instructions (planes by one
+// FMA each, widened for its rounding) gained 1 % and found hits that box_hit does not enter, for rays in the
+// plane of a box's face.
 constexpr int kRefill = 12;
 constexpr int kSplitIdle = 24;
 constexpr uint32_t kSplitEvery = 2;
